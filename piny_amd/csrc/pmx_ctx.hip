@@ -1345,12 +1345,13 @@ int build_ref_list(pmx_ctx *c) {
 }
 
 void add_stage(RedArgs &r, size_t off, int G, int nv, const std::vector<int> &slots) {
-  RedStage &st = r.st[r.nstage++];
+  RedStage &st = r.st[r.nstage];
   st.off = off;
   st.G = G;
   st.nv = nv;
   st.wv = 1.0;
-  for (int v = 0; v < nv; v++) st.slot[v] = slots[v];
+  for (int v = 0; v < nv; v++) r.row[slots[v]][r.nrow[slots[v]]++] = (unsigned char)(r.nstage | (v << 4));
+  r.nstage++;
 }
 
 IntraArgs intra_args(pmx_ctx *c, bool pimd) {
@@ -3310,12 +3311,9 @@ int pmx_get_param_grad(pmx_ctx *c, pmx_param_grad *out) {
     RedArgs red{};
     red.P = P;
     red.nslot = PAIRG_NV;
-    red.nstage = 1;
-    red.st[0].off = 0;
-    red.st[0].G = (int)gx;
-    red.st[0].nv = PAIRG_NV;
-    red.st[0].wv = 1.0;
-    for (int v = 0; v < PAIRG_NV; v++) red.st[0].slot[v] = v;
+    std::vector<int> slots(PAIRG_NV);
+    for (int v = 0; v < PAIRG_NV; v++) slots[v] = v;
+    add_stage(red, 0, (int)gx, PAIRG_NV, slots);
     red.part = c->gpart;
     red.acc = c->gacc;
     hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)P * PAIRG_NV + 1), dim3(256), 0, st, red);

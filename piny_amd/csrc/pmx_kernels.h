@@ -305,19 +305,21 @@ constexpr int INTRA_NV = 7;  // energy, 6 virial
 constexpr int FIN_NV = 10;   // 9 virial corrections, akvir
 constexpr int PAIRG_NV = 2 * MAX_LJ_GRAD;  // per LJ slot: energy per unit eps, sigma dV/dsigma per unit eps
 
-// One stage of partial sums: part[off + (g*P + b)*nv + v] for g < G holds
-// the contribution of block g to accumulator slot[v] of bead b.
+// One stage of partial sums: part[off + (v*P + b)*G + g] for g < G holds the
+// contribution of block g to the stage's value v of bead b.
 struct RedStage {
   size_t off;
   int G, nv;
-  int slot[12];
   double wv;  // weight of values 1 .. nv-1 (the virial of a RESPA-weighted stage), 1 otherwise
 };
 constexpr int MAX_RED_STAGES = 8;
+constexpr int MAX_RED_SLOTS = ACC_NUM;
 struct RedArgs {
   int P, nstage;
   int nslot;  // accumulator slots per bead (ACC_NUM for the energies)
   RedStage st[MAX_RED_STAGES];
+  // the rows that slot s sums, nrow[s] of them: stage | value << 4
+  unsigned char nrow[MAX_RED_SLOTS], row[MAX_RED_SLOTS][MAX_RED_STAGES];
   const double *part;
   double *acc;  // [P][nslot], every entry written
   // one scalar besides: *sacc = the sum of spart[0 .. sG) (0 when sG = 0),

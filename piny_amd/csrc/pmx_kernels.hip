@@ -28,11 +28,14 @@ __global__ void k_fill_double(double *p, double v, size_t n) {
 }
 
 // The per-bead sums from the partial rows: one workgroup per (bead, slot)
-// output (and one more for the scalar *sacc = the sum of spart[0 .. sG)),
-// its 256 lanes over the rows' entries, then a fixed-order tree in LDS, so
-// the result does not depend on timing.
+// output (and one more for the scalar *sacc = the sum of spart[0 .. sG)).
+// The slot's rows (a.row, matched on the host) are taken as one sequence, so
+// the loads of all of them are in flight together (row after row, each a
+// round trip to memory: 6.0 us for the shortest rows); the sums then go
+// through the wavefronts and LDS in a fixed order, so the result does not
+// depend on timing.
 __global__ void __launch_bounds__(256) k_reduce_partials(RedArgs a) {
-  __shared__ double red[256];
+  __shared__ double red[4];
   const int o = blockIdx.x, tid = threadIdx.x;
   const bool scalar = o == a.P * a.nslot;
   if (scalar && !a.sacc) return;  // uniform over the workgroup
@@ -40,32 +43,45 @@ __global__ void __launch_bounds__(256) k_reduce_partials(RedArgs a) {
   if (scalar) {
     for (int g = tid; g < a.sG; g += 256) s0 += a.spart[g];
   } else {
-    const int b = o / a.nslot, slot = o % a.nslot;
-    for (int si = 0; si < a.nstage; si++) {
-      const RedStage &r = a.st[si];
-      for (int v = 0; v < r.nv; v++) {
-        if (r.slot[v] != slot) continue;
-        const double *row = a.part + r.off + ((size_t)v * a.P + b) * r.G;
-        // a weight of 1 leaves every sum as it is (the products are exact)
-        const double w = v == 0 ? 1.0 : r.wv;
-        int g = tid;
-        for (; g + 256 < r.G; g += 512) {
-          s0 += w * row[g];
-          s1 += w * row[g + 256];
-        }
-        for (; g < r.G; g += 256) s0 += w * row[g];
-      }
+    const int b = o / a.nslot, slot = o % a.nslot, nr = a.nrow[slot];
+    const double *row[MAX_RED_STAGES];
+    int end[MAX_RED_STAGES];
+    double w[MAX_RED_STAGES];
+    int tot = 0;
+#pragma unroll
+    for (int r = 0; r < MAX_RED_STAGES; r++) {
+      const int rv = r < nr ? a.row[slot][r] : 0, v = rv >> 4;
+      const RedStage &st = a.st[rv & 15];
+      row[r] = a.part + st.off + ((size_t)v * a.P + b) * st.G - tot;
+      tot += r < nr ? st.G : 0;
+      end[r] = tot;
+      w[r] = v == 0 ? 1.0 : st.wv;  // a weight of 1 leaves every sum as it is (the products are exact)
     }
+    auto term = [&](int g) {
+      const double *p = row[0];
+      double wt = w[0];
+#pragma unroll
+      for (int r = 1; r < MAX_RED_STAGES; r++) {
+        p = g >= end[r - 1] ? row[r] : p;
+        wt = g >= end[r - 1] ? w[r] : wt;
+      }
+      return wt * p[g];
+    };
+    int g = tid;
+    for (; g + 768 < tot; g += 1024) {
+      const double t0 = term(g), t1 = term(g + 256), t2 = term(g + 512), t3 = term(g + 768);
+      s0 += t0 + t2;
+      s1 += t1 + t3;
+    }
+    for (; g < tot; g += 256) s0 += term(g);
   }
-  red[tid] = s0 + s1;
+  const double s = wave_sum_mod(s0 + s1, 1);
+  if ((tid & 63) == 0) red[tid >> 6] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if (tid < h) red[tid] += red[tid + h];
-    __syncthreads();
-  }
   if (tid == 0) {
-    if (scalar) *a.sacc = red[0];
-    else a.acc[(size_t)(o / a.nslot) * a.nslot + (o % a.nslot)] = red[0];
+    const double t = (red[0] + red[1]) + (red[2] + red[3]);
+    if (scalar) *a.sacc = t;
+    else a.acc[o] = t;
   }
 }
 
@@ -1891,10 +1907,23 @@ __global__ void __launch_bounds__(256) k_intra_mol(IntraArgs a) {
       a.fz[ib] = fl[(3 * s + 2) * bs + tid];
     }
   }
-  block_partials<INTRA_NV>(ae, a.P, 0, a.P, a.part_ecor, blockIdx.x, gridDim.x);
-  block_partials<INTRA_NV>(ab, a.P, 0, a.P, a.part_bond, blockIdx.x, gridDim.x);
-  block_partials<INTRA_NV>(aa, a.P, 0, a.P, a.part_bend, blockIdx.x, gridDim.x);
-  block_partials<FIN_NV>(cf, a.P, 0, a.P, a.part_fin, blockIdx.x, gridDim.x);
+  // the four stages' rows in one pass over the molecules' LDS, free by now
+  double vals[3 * INTRA_NV + FIN_NV];
+#pragma unroll
+  for (int k = 0; k < INTRA_NV; k++) {
+    vals[k] = ae[k];
+    vals[INTRA_NV + k] = ab[k];
+    vals[2 * INTRA_NV + k] = aa[k];
+  }
+#pragma unroll
+  for (int k = 0; k < FIN_NV; k++) vals[3 * INTRA_NV + k] = cf[k];
+  __syncthreads();
+  block_sums<3 * INTRA_NV + FIN_NV>(vals, a.P, lds_mol, 2 * R * bs, [&](int k, int b, double t) {
+    const int st = k / INTRA_NV;  // 3 and beyond: the finish stage
+    double *part = st == 0 ? a.part_ecor : st == 1 ? a.part_bond : st == 2 ? a.part_bend : a.part_fin;
+    const int v = st < 3 ? k - st * INTRA_NV : k - 3 * INTRA_NV;
+    part[((size_t)v * a.P + b) * gridDim.x + blockIdx.x] = t;
+  });
 }
 
 // ---------------------------------------------------------------------------
