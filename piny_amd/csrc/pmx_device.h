@@ -132,16 +132,24 @@ __device__ __forceinline__ void block_partials(const double (&v)[NV], int nb, in
 // Workgroups are dispatched to the 8 XCDs of an MI355X in turn (workgroup
 // id modulo 8), each XCD with its own L2.  Kernels whose work is (unit,
 // bead) with units sharing a bead's data (PME tiles, FFT planes) launch
-// 8 * units * ceil(P/8) workgroups in one dimension and map them so that
-// every unit of one bead runs on one XCD.  Returns false for the padding
-// workgroups of the last bead group.
-__device__ __forceinline__ bool xcd_unit_bead(int units, int P, int &unit, int &bead) {
-  const int L = blockIdx.x, x = L & 7, r = L >> 3;
-  bead = x + 8 * (r / units);
-  unit = r % units;
-  return bead < P;
+// units * P workgroups in one dimension.  Every group of 8 beads puts one
+// bead on each XCD, so a bead's data stays in one L2.  The P % 8 beads left
+// over are dealt to all XCDs, beads fastest: one XCD a bead would leave the
+// others idle (a box of one bead ran its k space on 32 of the 256 CUs; 5003
+// SPC/Fw, P = 1: 329 -> 309 us a force call).
+__device__ __forceinline__ void xcd_unit_bead(int units, int P, int &unit, int &bead) {
+  const int L = blockIdx.x, full = P & ~7, nfull = units * full;
+  if (L < nfull) {
+    const int r = L >> 3;
+    bead = (L & 7) + 8 * (r / units);
+    unit = r % units;
+  } else {
+    const int r = L - nfull, rem = P - full;
+    bead = full + r % rem;
+    unit = r / rem;
+  }
 }
 
-inline unsigned xcd_grid(int units, int P) { return 8u * (unsigned)units * (unsigned)((P + 7) / 8); }
+inline unsigned xcd_grid(int units, int P) { return (unsigned)units * (unsigned)P; }
 
 }  // namespace pmx

@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(spread_lanes<T>() * PME_BLOCK) k_pme_spread(Pm
   double *box = (double *)lds_raw;
   const int hvol = (int)a.hvol;
   int tl, b;
-  if (!xcd_unit_bead(a.ntile, a.P, tl, b)) return;  // uniform over the workgroup
+  xcd_unit_bead(a.ntile, a.P, tl, b);
   const int tid = threadIdx.x;
   for (int k = tid; k < hvol; k += blockDim.x) box[k] = 0.0;
   const size_t bin = (size_t)b * a.ntile + tl;
@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T *box = (T *)lds_raw;
   int tl, b;
-  if (!xcd_unit_bead(a.ntile, a.P, tl, b)) return;
+  xcd_unit_bead(a.ntile, a.P, tl, b);
   const int tid = threadIdx.x;
   const size_t bin = (size_t)b * a.ntile + tl;
   const int lo = a.bin_off[bin], cnt = a.bin_cnt[bin];
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(PME_BLOCK) k_pme_phi(PmeArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T *box = (T *)lds_raw;
   int tl, b;
-  if (!xcd_unit_bead(a.ntile, a.P, tl, b)) return;
+  xcd_unit_bead(a.ntile, a.P, tl, b);
   const int tid = threadIdx.x;
   const size_t bin = (size_t)b * a.ntile + tl;
   const int lo = a.bin_off[bin], cnt = a.bin_cnt[bin];
@@ -922,7 +922,7 @@ __global__ void __launch_bounds__(NT) k_fft_fwd_ab(FftArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   C *sm = (C *)lds_raw;
   int c, b;
-  if (!xcd_unit_bead(a.K[2], a.P, c, b)) return;
+  xcd_unit_bead(a.K[2], a.P, c, b);
   const int Ka = a.K[0], Kb = a.K[1], Ha = Ka / 2 + 1;
   C *twa = sm + Ka * Kb, *twb = twa + Ka;  // twiddles after the plane
   stage_twiddles<T>(a, 0, twa);
@@ -954,7 +954,7 @@ __global__ void __launch_bounds__(NT) k_fft_c_conv(FftArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   C *sm = (C *)lds_raw;
   int bb, b;
-  if (!xcd_unit_bead(a.K[1], a.P, bb, b)) return;
+  xcd_unit_bead(a.K[1], a.P, bb, b);
   const int Ka = a.K[0], Kb = a.K[1], Kc = a.K[2], Ha = Ka / 2 + 1;
   C *twc = sm + Kc * Ha;  // twiddles after the lines
   stage_twiddles<T>(a, 2, twc);
@@ -1031,7 +1031,7 @@ __global__ void __launch_bounds__(NT) k_fft_inv_ba(FftArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   C *sm = (C *)lds_raw;
   int c, b;
-  if (!xcd_unit_bead(a.K[2], a.P, c, b)) return;
+  xcd_unit_bead(a.K[2], a.P, c, b);
   const int Ka = a.K[0], Kb = a.K[1], Ha = Ka / 2 + 1;
   C *twa = sm + Ka * Kb, *twb = twa + Ka;  // twiddles after the plane
   stage_twiddles<T>(a, 0, twa);
