@@ -93,7 +93,7 @@ struct pmx_ctx {
   int *b1 = nullptr, *b2 = nullptr, *btyp = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr,
       *atyp = nullptr, *e1 = nullptr, *e2 = nullptr;
   double *bc = nullptr, *beq = nullptr, *ac = nullptr, *as = nullptr;
-  int nghost = 0, *gatom = nullptr, *gncomp = nullptr, *gcomp = nullptr;
+  int nghost = 0, *gatom = nullptr, *gncomp = nullptr, *gcomp = nullptr, *gsite = nullptr;  // gsite: ghost of a site, -1
   std::vector<int> ghost_h;  // the ghost sites (host copy)
   // molecules of k_intra_mol (nmol = 0: the topology does not split into
   // molecules of at most MOL_MAX consecutive sites; per-term kernels then)
@@ -929,7 +929,7 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
   TRY(dalloc(c, &c->x, NP));
   TRY(dalloc(c, &c->y, NP));
   TRY(dalloc(c, &c->z, NP));
-  TRY(dalloc(c, &c->stage, NP));
+  TRY(dalloc(c, &c->stage, 3 * NP));
   TRY(dalloc(c, &c->fx, NP));
   TRY(dalloc(c, &c->fy, NP));
   TRY(dalloc(c, &c->fz, NP));
@@ -1051,6 +1051,11 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
   c->nghost = sys->nghost;
   c->ghost_h.assign(sys->ghost_atom, sys->ghost_atom + sys->nghost);
   TRY(upload(c, &c->gatom, sys->ghost_atom, sys->nghost));
+  if (sys->nghost) {
+    std::vector<int> gs(N, -1);
+    for (int g = 0; g < sys->nghost; g++) gs[sys->ghost_atom[g]] = g;
+    TRY(upload(c, &c->gsite, gs.data(), N));
+  }
   TRY(upload(c, &c->gncomp, sys->ghost_ncomp, sys->nghost));
   TRY(upload(c, &c->gcomp, sys->ghost_comp, (size_t)4 * sys->nghost));
   TRY(upload(c, &c->gcoef, sys->ghost_coef, (size_t)4 * sys->nghost));
@@ -2183,23 +2188,52 @@ void pmx_destroy(pmx_ctx *c) {
 
 const char *pmx_last_error(const pmx_ctx *c) { return c ? c->err.c_str() : "null context"; }
 
-static int set_pos_common(pmx_ctx *c, const double *x, const double *y, const double *z, hipMemcpyKind kind) {
-  Setup &s = c->s;
-  const size_t NP = (size_t)s.N * s.P;
-  HIPCHK(hipSetDevice(c->device));
+// n doubles at p lie in one allocation of this device, so a kernel may read them
+static bool device_readable(const pmx_ctx *c, const double *p, size_t n) {
+  hipPointerAttribute_t at{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != c->device ||
+      hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return ((uintptr_t)p & 7) == 0 && (const char *)p + n * sizeof(double) <= (const char *)base + size;
+}
+
+// Bead-major x, y, z (host or device) into the atom-major dst arrays: device
+// arrays are read where they are, others through the staging buffer; one
+// kernel for the three.  Returns once the sources have been read.
+static int to_atom_major(pmx_ctx *c, const double *x, const double *y, const double *z, double *const dst[3],
+                         hipMemcpyKind kind, bool ghosts) {
+  const size_t NP = (size_t)c->s.N * c->s.P;
   const double *src[3] = {x, y, z};
-  double *dst[3] = {c->x, c->y, c->z};
+  Layout3 a{};
+  a.N = c->s.N;
+  a.P = c->s.P;
+  a.to_atom = 1;
   for (int d = 0; d < 3; d++) {
-    HIPCHK(hipMemcpyAsync(c->stage, src[d], NP * sizeof(double), kind, c->st));
-    hipLaunchKernelGGL(k_bead_to_atom, dim3(blocks(NP)), dim3(256), 0, c->st, s.N, s.P, c->stage, dst[d]);
-    HIPCHK(hipGetLastError());
+    a.dst[d] = dst[d];
+    a.src[d] = src[d];
+    if (kind == hipMemcpyDeviceToDevice && device_readable(c, src[d], NP)) continue;
+    a.src[d] = c->stage + d * NP;
+    HIPCHK(hipMemcpyAsync(c->stage + d * NP, src[d], NP * sizeof(double), kind, c->st));
   }
-  if (c->nghost) {
-    hipLaunchKernelGGL(k_ghost_pos, dim3(blocks((size_t)c->nghost * s.P)), dim3(256), 0, c->st, c->nghost, s.P,
-                       c->gatom, c->gncomp, c->gcomp, c->gcoef, c->x, c->y, c->z);
-    HIPCHK(hipGetLastError());
+  if (ghosts && c->nghost) {
+    a.ghost = c->gsite;
+    a.gncomp = c->gncomp;
+    a.gcomp = c->gcomp;
+    a.gcoef = c->gcoef;
   }
+  HIPCHK(launch_layout3(a, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
+  return PMX_OK;
+}
+
+static int set_pos_common(pmx_ctx *c, const double *x, const double *y, const double *z, hipMemcpyKind kind) {
+  HIPCHK(hipSetDevice(c->device));
+  double *const dst[3] = {c->x, c->y, c->z};
+  if (int rc = to_atom_major(c, x, y, z, dst, kind, true)) return rc;
   c->have_pos = true;
   c->grad_ready = false;
   return PMX_OK;
@@ -2731,20 +2765,29 @@ int pmx_batch_autotune(pmx_batch *b, unsigned flags, int reps, int *choice) {
   return pmx_batch_energy_control(b, flags, out.data());
 }
 
+// three atom-major arrays into host memory, bead-major
+static int get_bead_major(pmx_ctx *c, double *const src[3], double *fx, double *fy, double *fz) {
+  const size_t NP = (size_t)c->s.N * c->s.P;
+  HIPCHK(hipSetDevice(c->device));
+  double *dst[3] = {fx, fy, fz};
+  Layout3 a{};
+  a.N = c->s.N;
+  a.P = c->s.P;
+  for (int d = 0; d < 3; d++) {
+    a.src[d] = src[d];
+    a.dst[d] = c->stage + d * NP;
+  }
+  HIPCHK(launch_layout3(a, c->st));
+  for (int d = 0; d < 3; d++)
+    HIPCHK(hipMemcpyAsync(dst[d], c->stage + d * NP, NP * sizeof(double), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  return PMX_OK;
+}
+
 int pmx_get_forces(pmx_ctx *c, double *fx, double *fy, double *fz) {
   if (!c || !fx || !fy || !fz) return PMX_ERR_ARG;
-  Setup &s = c->s;
-  const size_t NP = (size_t)s.N * s.P;
-  HIPCHK(hipSetDevice(c->device));
   double *src[3] = {c->fx, c->fy, c->fz};
-  double *dst[3] = {fx, fy, fz};
-  for (int d = 0; d < 3; d++) {
-    hipLaunchKernelGGL(k_atom_to_bead, dim3(blocks(NP)), dim3(256), 0, c->st, s.N, s.P, src[d], c->stage);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dst[d], c->stage, NP * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-  }
-  return PMX_OK;
+  return get_bead_major(c, src, fx, fy, fz);
 }
 
 int pmx_get_forces_device(pmx_ctx *c, const double **fx, const double **fy, const double **fz) {
@@ -2752,20 +2795,6 @@ int pmx_get_forces_device(pmx_ctx *c, const double **fx, const double **fy, cons
   *fx = c->fx;
   *fy = c->fy;
   *fz = c->fz;
-  return PMX_OK;
-}
-
-static int get_bead_major(pmx_ctx *c, double *const src[3], double *fx, double *fy, double *fz) {
-  Setup &s = c->s;
-  const size_t NP = (size_t)s.N * s.P;
-  HIPCHK(hipSetDevice(c->device));
-  double *dst[3] = {fx, fy, fz};
-  for (int d = 0; d < 3; d++) {
-    hipLaunchKernelGGL(k_atom_to_bead, dim3(blocks(NP)), dim3(256), 0, c->st, s.N, s.P, src[d], c->stage);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dst[d], c->stage, NP * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-  }
   return PMX_OK;
 }
 
@@ -2788,17 +2817,8 @@ int pmx_get_fxt(pmx_ctx *c, double *fx, double *fy, double *fz) {
 }
 
 static int set_bead_major(pmx_ctx *c, double *const dst[3], const double *x, const double *y, const double *z) {
-  Setup &s = c->s;
-  const size_t NP = (size_t)s.N * s.P;
   HIPCHK(hipSetDevice(c->device));
-  const double *src[3] = {x, y, z};
-  for (int d = 0; d < 3; d++) {
-    HIPCHK(hipMemcpyAsync(c->stage, src[d], NP * sizeof(double), hipMemcpyHostToDevice, c->st));
-    hipLaunchKernelGGL(k_bead_to_atom, dim3(blocks(NP)), dim3(256), 0, c->st, s.N, s.P, c->stage, dst[d]);
-    HIPCHK(hipGetLastError());
-  }
-  HIPCHK(hipStreamSynchronize(c->st));
-  return PMX_OK;
+  return to_atom_major(c, x, y, z, dst, hipMemcpyHostToDevice, false);
 }
 
 int pmx_set_velocities(pmx_ctx *c, const double *vx, const double *vy, const double *vz) {

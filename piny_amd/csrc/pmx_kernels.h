@@ -329,7 +329,16 @@ struct RedArgs {
   double *sacc;
 };
 
-__global__ void k_bead_to_atom(int N, int P, const double *src, double *dst);
+// x, y and z between the bead-major and the atom-major order; ghost: per site
+// the ghost it is, or -1 (null: the sites are copied as they are)
+struct Layout3 {
+  int N, P, to_atom, TS;
+  const double *src[3];
+  double *dst[3];
+  const int *ghost, *gncomp, *gcomp;
+  const double *gcoef;
+};
+hipError_t launch_layout3(Layout3 a, hipStream_t st);
 __global__ void k_atom_to_bead(int N, int P, const double *src, double *dst);
 __global__ void k_ghost_pos(int ng, int P, const int *gatom, const int *gncomp, const int *gcomp,
                             const double *gcoef, double *x, double *y, double *z);

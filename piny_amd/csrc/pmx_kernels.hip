@@ -88,18 +88,56 @@ __global__ void __launch_bounds__(256) k_reduce_partials(RedArgs a) {
 // ---------------------------------------------------------------------------
 // layout conversion
 
-__global__ void k_bead_to_atom(int N, int P, const double *__restrict__ src, double *__restrict__ dst) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)N * P) return;
-  const int i = (int)(t / P), b = (int)(t % P);
-  dst[t] = src[(size_t)b * N + i];
-}
-
 __global__ void k_atom_to_bead(int N, int P, const double *__restrict__ src, double *__restrict__ dst) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (size_t)N * P) return;
   const int b = (int)(t / N), i = (int)(t % N);
   dst[t] = src[(size_t)i * P + b];
+}
+
+// Three arrays at once between PINY's bead-major order and the atom-major one
+// (to_atom says which way), a tile of TS sites and all their beads per
+// workgroup through LDS, so that both sides move whole runs: P doubles a site
+// on the atom-major side, TS a bead on the other.  With a ghost map (to_atom)
+// the ghost sites' rows are formed from the source in the same pass
+// (get_ghost_pos, ghost_control.c:28-64: same summation order, no FMA).
+__global__ void __launch_bounds__(256) k_layout3(Layout3 a) {
+#pragma clang fp contract(off)
+  extern __shared__ double tile[];  // [3][TS][P + 1]
+  const int P = a.P, N = a.N, i0 = blockIdx.x * a.TS, n = min(a.TS, N - i0), ld = P + 1, vol = a.TS * ld;
+  for (int t = threadIdx.x; t < n * P; t += blockDim.x) {
+    const int s = a.to_atom ? t % n : t / P, b = a.to_atom ? t / n : t % P;
+    const size_t g = a.to_atom ? (size_t)b * N + i0 + s : (size_t)(i0 + s) * P + b;
+#pragma unroll
+    for (int d = 0; d < 3; d++) tile[d * vol + s * ld + b] = a.src[d][g];
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < n * P; t += blockDim.x) {
+    const int s = a.to_atom ? t / P : t % n, b = a.to_atom ? t % P : t / n;
+    const size_t g = a.to_atom ? (size_t)(i0 + s) * P + b : (size_t)b * N + i0 + s;
+    const int gh = a.ghost ? a.ghost[i0 + s] : -1;
+    if (gh < 0) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) a.dst[d][g] = tile[d * vol + s * ld + b];
+    } else {
+      double r[3] = {0.0, 0.0, 0.0};
+      for (int k = 0; k < a.gncomp[gh]; k++) {
+        const size_t ia = (size_t)b * N + a.gcomp[4 * gh + k];
+        const double c = a.gcoef[4 * gh + k];
+#pragma unroll
+        for (int d = 0; d < 3; d++) r[d] += c * a.src[d][ia];
+      }
+#pragma unroll
+      for (int d = 0; d < 3; d++) a.dst[d][g] = r[d];
+    }
+  }
+}
+
+hipError_t launch_layout3(Layout3 a, hipStream_t st) {
+  a.TS = a.P >= 16 ? 16 : 256 / a.P;  // at least 256 items a workgroup; 26 KB of LDS at P = 64
+  const size_t lds = (size_t)3 * a.TS * (a.P + 1) * sizeof(double);
+  hipLaunchKernelGGL(k_layout3, dim3((a.N + a.TS - 1) / a.TS), dim3(256), lds, st, a);
+  return hipGetLastError();
 }
 
 // get_ghost_pos, ghost_control.c:28-64 (same summation order, no FMA)

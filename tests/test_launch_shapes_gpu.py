@@ -38,3 +38,29 @@ def check(c, **kw):
 @pytest.mark.parametrize("P", [1, 2, 3, 6, 12, 40, 48, 64])
 def test_partial_sums_per_bead_count(P):
     check(w.small_config(w.Q_TIP4P_F, nmol=30, P=P, seed=40 + P))
+
+
+# tiles of the layout change: whole ones and a remainder, few and many beads
+@pytest.mark.parametrize("nmol, P", [(2, 1), (64, 1), (65, 3), (4, 16), (7, 24), (33, 64)])
+def test_positions_in_and_out(nmol, P):
+    import torch
+    from piny_amd.engine import Engine
+    c = w.small_config(w.Q_TIP4P_F, nmol=nmol, P=P, seed=3)
+    x = np.stack([v.reshape(P, -1) for v in (c.x, c.y, c.z)], 2)
+    m = w.Q_TIP4P_F
+    xg = x.reshape(P, nmol, 4, 3).copy()
+    xg[:, :, 3] = sum(cf * xg[:, :, k] for k, cf in m.ghost[1])
+    eng = Engine(c.system, c.x, c.y, c.z)
+    eng.set_positions(c.x, c.y, c.z)
+    host = eng.positions()
+    eng.set_velocities(c.y, c.z, c.x)
+    assert np.array_equal(eng.velocities(), x[:, :, [1, 2, 0]])
+    dev = [torch.as_tensor(v, device="cuda") for v in (c.x, c.y, c.z)]
+    torch.cuda.synchronize()
+    eng.set_positions(c.x * 0.0, c.y, c.z)
+    eng.set_positions_device(*[v.data_ptr() for v in dev])
+    assert np.array_equal(eng.positions(), host)
+    real = np.arange(4 * nmol) % 4 != 3
+    assert np.array_equal(host[:, real], x[:, real])
+    assert np.abs(host.reshape(P, nmol, 4, 3) - xg).max() < 1e-12
+    eng.close()
