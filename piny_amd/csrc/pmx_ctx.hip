@@ -64,6 +64,7 @@ struct pmx_ctx {
   double4 *site = nullptr;     // [N] (xmod, q)
   float4 *disp = nullptr;      // mixed precision with beads: x - xmod in FP32 [N*P]
   double *umax = nullptr;      // the largest |x - xmod| of every site over its beads [N]
+  bool one_tab = false;    // FP64 tables: every type pair has the same erfc table, which fits a workgroup's LDS
   int pair_mode = 0;       // 0 FP64 tables, 1 FP64 direct, 2 FP32 direct
   // molecule-cluster form of the mixed pair kernel (k_pair_clu)
   bool clu_ok = false;      // the box qualifies: one molecule template of <= 4 sites, one cutoff
@@ -986,6 +987,9 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
     TRY(upload(c, &c->pair_pp_res, ppr.data(), ppr.size()));
     TRY(dalloc(c, &c->site, N));
     c->pair_mode = (c->par.precision == PMX_PREC_MIXED) ? 2 : (c->par.pair_eval == PMX_PAIR_DIRECT ? 1 : 0);
+    c->one_tab = c->pair_mode == 0 && pair_tab_lds_fits(s.nsplin) && NP * sizeof(double) <= (size_t)UINT32_MAX;
+    for (int t = 1; t < s.npair; t++)
+      c->one_tab = c->one_tab && s.rmin[t] == s.rmin[0] && s.cutoff[t] == s.cutoff[0];
     if (c->pair_mode == 2 && P > 1) {
       if (NP * sizeof(float4) > (size_t)UINT32_MAX) {  // the pair kernel reads them at 32-bit byte offsets
         set_err(c, "%d sites x %d beads exceed the 2^28 bead displacements of the mixed precision", N, P);
@@ -1751,8 +1755,18 @@ int main_sequence(pmx_ctx *c, unsigned flags, hipStream_t st, bool timing) {
     a.fy = c->fy;
     a.fz = c->fz;
     a.part = c->part + c->off_pair;
+    if (c->pair_mode == 0 && c->full_list && c->one_tab) {
+      a.wps = pair_tab_wps(N);
+      a.gx = pair_tab_grid_x(N, c->pair_waves);
+      a.t_cut = s.cutoff[0];
+      a.t_rmin = s.rmin[0];
+      a.t_dri = s.dri[0];
+      a.cullv = a.pp == c->pair_pp_res;
+      for (int t = 0; t < s.npair; t++)
+        if (s.label[t] == PMX_INTER_LJ) a.ljmask |= 1ull << t;
+    }
     HIPCHK(launch_pair(a, c->pair_mode, c->full_list, st));
-    add_stage(red, c->off_pair, pair_grid_x(N, c->pair_waves), PAIR_NV,
+    add_stage(red, c->off_pair, a.gx, PAIR_NV,
               {ACC_VVDW, ACC_VCOUL, ACC_P11, ACC_P22, ACC_P33, ACC_P12, ACC_P13, ACC_P23, ACC_NPAIR});
   }
   if (c->pme_deferred) {

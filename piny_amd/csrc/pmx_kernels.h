@@ -83,6 +83,12 @@ struct PairArgs {
   int nftab;
   int2 ftoff[MAX_PAIRS];
   int swit;
+  // the FP64 table kernel with its erfc table in LDS (wps > 0: wavefronts per
+  // site): the one grid and cutoff of every type pair, the type pairs with an
+  // LJ term, and whether their culling radii differ (RESPA cutoffs)
+  int wps, cullv;
+  double t_cut, t_rmin, t_dri;
+  unsigned long long ljmask;
   // RESPA: one of RESPA_*, the weights of the full and the short-range
   // forces (the switch runs over rheal below PP_CUTRES)
   int respa;
@@ -458,6 +464,9 @@ hipError_t launch_pair_clu(const CluArgs &a, int gx, hipStream_t st);
 
 hipError_t launch_pair_grad(const PairArgs &a, int mode, hipStream_t st);
 int pair_grid_x(int N, int max_waves);
+bool pair_tab_lds_fits(int nsplin);
+int pair_tab_wps(int N);
+int pair_tab_grid_x(int N, int max_waves);
 constexpr int PAIR_MAX_WAVES = 16384;  // the largest pair grid the autotuner tries
 // LDS bytes of the spread and gather workgroups for a given tiling
 size_t pme_lds_bytes(const PmeArgs &a, bool gather);

@@ -1547,6 +1547,227 @@ __global__ void __launch_bounds__(256) k_pair_staged_dir(PairArgs a) {
   pair_staged<B, 1>(a);
 }
 
+// V and -V'/r of one table at fractional offset del from point k (0-based):
+// the cubic of spline4 (Lagrange's through points k - 2 .. k + 1) as four
+// weights that serve both functions.
+__device__ __forceinline__ double2 spline4_both(const double2 *tab, int k, double del) {
+  const double2 tm2 = tab[k - 2], tm1 = tab[k - 1], t0 = tab[k], tp1 = tab[k + 1];
+  const double a = del + 1.0, b = del + 2.0, c = del - 1.0, ab = a * b, dc = del * c;
+  const double w1 = (1.0 / 6.0) * (del * ab), w0 = -0.5 * (c * ab), wm1 = 0.5 * (dc * b), wm2 = (-1.0 / 6.0) * (dc * a);
+  return make_double2(wm2 * tm2.x + wm1 * tm1.x + w0 * t0.x + w1 * tp1.x,
+                      wm2 * tm2.y + wm1 * tm1.y + w0 * t0.y + w1 * tp1.y);
+}
+
+// sqrt(x) for normal x > 0: v_rsq_f64, one coupled Newton step for the root
+// and half its reciprocal, then the root's residual once more; within an ulp
+// of the correctly rounded root, which costs twice the instructions (scaling
+// for the ends of the exponent range).  x = 0 gives NaN, infinities too.
+__device__ __forceinline__ double sqrt_normal(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
+// pair_staged with tables (MODE 0) for systems whose type pairs share one
+// erfc table (one spline start and cutoff): workgroups of 16 wavefronts, one
+// a CU, hold that table in LDS (80 KB at 5000 points); LJ tables stay in
+// memory (one pair in ten, and a branch).  Read through the caches the
+// table's gathers were the bound: every lane of a term takes 64 bytes at its
+// own place of a table larger than the L1, about 180 bytes of lines each
+// (4096 q-TIP4P/F, P = 32: 911 us at 47 % VALU busy, 785 us with the table
+// in LDS).  The kernel then issues FP64 instructions: 109 a term, of which
+// the correctly rounded root, the interpolation's coefficients per function,
+// 64-bit addresses and the index's integer round trip were 40 (spline4_both,
+// sqrt_normal, byte offsets staged with the entries): TIMEUS us.
+//
+// a.wps wavefronts share a site, taking its row's chunks in turn, and add
+// their forces through LDS: with fewer sites than the 4096 wavefronts the
+// chip holds, a row's dependent reads are the kernel's time.
+constexpr int TAB_WAVES = 16;
+template <int B, bool PIMD>
+__global__ void __launch_bounds__(64 * TAB_WAVES) k_pair_tab_lds(PairArgs a) {
+  constexpr int S = 64 / B;
+  // the pair loop loads positions up to 4 S entries past a chunk's end
+  constexpr int SPAD = PIMD ? 64 + 4 * S : 1;
+  __shared__ double scr[MAX_PAIRS];  // RESPA cutoff per type pair
+  __shared__ double4 sdf[TAB_WAVES][64];
+  __shared__ int styp[TAB_WAVES][64];  // type pair, negative (~t) without an LJ term
+  // byte offset of site j's first bead position per staged entry, 0 past the
+  // chunk's end (a valid address whose value goes unused)
+  __shared__ unsigned soff[TAB_WAVES][SPAD];
+  extern __shared__ double2 stab[];  // [nsplin]
+  for (int k = threadIdx.x; k < a.npair; k += blockDim.x) scr[k] = a.pp[k * PP_NUM + PP_CUTRES];
+  for (int k = threadIdx.x; k < a.nsplin; k += blockDim.x) stab[k] = a.tab_c[k];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (PIMD)
+    for (int k = 64 + lane; k < SPAD; k += 64) soff[w][k] = 0u;
+  __syncthreads();
+  const int slot = lane / B;
+  const int bead = (lane % B) + blockIdx.y * B;
+  const bool bact = bead < a.P;
+  const int P = a.P, W = a.wps, part = w % W;
+  const Cell &c = a.cell;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const double cut = a.t_cut, rmin = a.t_rmin, dri = a.t_dri;
+  const double cull = a.pp[PP_CULL];
+  const unsigned boff = (unsigned)(bact ? bead : 0) * (unsigned)sizeof(double);
+  PairAcc s{};
+  int npr = 0;
+  const int spb = TAB_WAVES / W;  // sites per workgroup and round
+  for (int i0 = blockIdx.x * spb; i0 < a.N; i0 += gridDim.x * spb) {
+    const int i = i0 + w / W;
+    const size_t ib = (size_t)min(i, a.N - 1) * P + (bact ? bead : 0);
+    double fxi = 0.0, fyi = 0.0, fzi = 0.0;
+    if (i < a.N) {
+      const double4 si = a.site[i];
+      double uix = 0.0, uiy = 0.0, uiz = 0.0;
+      if (PIMD) {
+        uix = a.x[ib] - si.x;
+        uiy = a.y[ib] - si.y;
+        uiz = a.z[ib] - si.z;
+      }
+      const int cnt = a.cnt[i];
+      const int *row = a.jlist + (size_t)i * a.cap;
+      s.fx = s.fy = s.fz = 0.0;
+      int enext = part * 64 + lane < cnt ? row[part * 64 + lane] : 0;
+      for (int k0 = part * 64; k0 < cnt; k0 += 64 * W) {
+        const int ks = k0 + lane, e = enext;
+        enext = ks + 64 * W < cnt ? row[ks + 64 * W] : 0;
+        bool keep = false;
+        double dx = 0.0, dy = 0.0, dz = 0.0, q2 = 0.0;
+        if (ks < cnt) {
+          const int j = e & ENTRY_MASK;
+          const double4 sj = a.site[j];
+          double lim = a.cullv ? a.pp[(e >> ENTRY_SHIFT) * PP_NUM + PP_CULL] : cull;
+          if (PIMD) {
+            min_image_sep(c, 1, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, si.x, si.y, si.z, sj.x, sj.y, sj.z, dx, dy, dz);
+            dx += si.x - sj.x;
+            dy += si.y - sj.y;
+            dz += si.z - sj.z;
+            lim = (lim + a.umax[i] + a.umax[j]) * (1.0 + 1e-9);
+            keep = dx * dx + dy * dy + dz * dz < lim * lim;
+            dx += sj.x;  // F = D + xmod_j
+            dy += sj.y;
+            dz += sj.z;
+          } else {
+            min_image_sep(c, 0, a.x[i], a.y[i], a.z[i], a.x[j], a.y[j], a.z[j], 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, dx,
+                          dy, dz);
+            lim *= 1.0 + 1e-9;
+            keep = dx * dx + dy * dy + dz * dz < lim * lim;
+          }
+          q2 = si.w * sj.w;
+        }
+        const uint64_t mk = __ballot(keep);
+        const int nk = __popcll(mk);
+        if (keep) {
+          const int pos = __popcll(mk & below), t = e >> ENTRY_SHIFT;
+          sdf[w][pos] = make_double4(dx, dy, dz, q2);
+          styp[w][pos] = (a.ljmask >> t) & 1ull ? t : ~t;
+          if (PIMD) soff[w][pos] = (unsigned)(e & ENTRY_MASK) * (unsigned)P * (unsigned)sizeof(double);
+        }
+        if (PIMD && lane >= nk) soff[w][lane] = 0u;
+        wave_sync();
+        auto pos = [&](int p) {
+          double3 r = make_double3(0.0, 0.0, 0.0);
+          if (PIMD) {  // 32-bit byte offsets from the kernel arguments
+            const unsigned o = soff[w][p] + boff;
+            r.x = *(const double *)((const char *)a.x + o);
+            r.y = *(const double *)((const char *)a.y + o);
+            r.z = *(const double *)((const char *)a.z + o);
+          }
+          return r;
+        };
+        auto pair = [&](int p, const double3 &xj) {
+          const double4 f = sdf[w][p];
+          double rx = f.x, ry = f.y, rz = f.z;
+          if (PIMD) {
+            rx = uix + (f.x - xj.x);
+            ry = uiy + (f.y - xj.y);
+            rz = uiz + (f.z - xj.z);
+          }
+          const double rd = sqrt_normal(rx * rx + ry * ry + rz * rz);
+          if (!bact || !(rd < cut)) return;
+          const int t = styp[w][p];
+          // the nearest point of the grid and the offset from it; rd < cut
+          // keeps the point below nsplin - 2
+          const double u = (rd - rmin) * dri, kd = fmax(rint(u), 0.0), del = u - kd;
+          const int k = (int)kd + 2;
+          double dvd = 0.0;
+          if (t >= 0) {
+            const double2 v = spline4_both(a.tab_lj + (size_t)t * a.nsplin, k, del);
+            s.vlj += v.x;
+            dvd += v.y;
+          }
+          if (f.w != 0.0) {
+            const double2 v = spline4_both(stab, k, del);
+            s.vc += f.w * v.x;
+            dvd += f.w * v.y;
+          }
+          if (a.respa) dvd *= respa_weight(a, scr[t >= 0 ? t : ~t], rd);  // uniform over the launch
+          const double fx1 = rx * dvd, fy1 = ry * dvd, fz1 = rz * dvd;
+          s.fx += fx1;
+          s.fy += fy1;
+          s.fz += fz1;
+          s.p11 += rx * fx1;
+          s.p22 += ry * fy1;
+          s.p33 += rz * fz1;
+          s.p12 += rx * fy1;
+          s.p13 += rx * fz1;
+          s.p23 += ry * fz1;
+          npr++;
+        };
+        // two pairs per iteration, each position loaded a whole iteration
+        // ahead into registers of its own, on every path (see k_pair_mixed)
+        double3 xA = pos(slot), xB = pos(slot + S);
+        int p = slot;
+        for (; p + S < nk; p += 2 * S) {
+          pair(p, xA);
+          xA = pos(p + 2 * S);
+          pair(p + S, xB);
+          xB = pos(p + 3 * S);
+        }
+        if (p < nk) pair(p, xA);
+        wave_sync();
+      }
+      fxi = wave_sum_mod(s.fx, B);
+      fyi = wave_sum_mod(s.fy, B);
+      fzi = wave_sum_mod(s.fz, B);
+    }
+    if (W > 1) {  // uniform over the launch
+      double *sf = (double *)sdf[w];  // 3 x 64, this wavefront's staging slice
+      if (slot == 0) {
+        sf[lane] = fxi;
+        sf[64 + lane] = fyi;
+        sf[128 + lane] = fzi;
+      }
+      __syncthreads();
+      if (part == 0 && slot == 0)
+        for (int q = 1; q < W; q++) {
+          const double *so = (const double *)sdf[w + q];
+          fxi += so[lane];
+          fyi += so[64 + lane];
+          fzi += so[128 + lane];
+        }
+      __syncthreads();
+    }
+    if (i < a.N && part == 0 && slot == 0 && bact) {  // the first writer of this step's forces
+      a.fx[ib] = fxi;
+      a.fy[ib] = fyi;
+      a.fz[ib] = fzi;
+    }
+  }
+  __syncthreads();  // the table's LDS is free for the sums
+  double vals[PAIR_NV] = {s.vlj * 0.5, s.vc * 0.5, s.p11 * 0.5, s.p22 * 0.5, s.p33 * 0.5,
+                          s.p12 * 0.5, s.p13 * 0.5, s.p23 * 0.5, (double)npr * 0.5};
+  block_sums<PAIR_NV>(vals, B, (double *)stab, 2 * a.nsplin, [&](int k, int b, double t) {
+    const int bd = (int)blockIdx.y * B + b;
+    if (bd < P) a.part[((size_t)k * P + bd) * gridDim.x + blockIdx.x] = t;
+  });
+}
+
 // The largest |x - xmod| of every site over its beads, in FP64 (one thread
 // per site), for the FP64 staged kernel's culling.
 __global__ void k_site_umax64(int N, int P, const double *__restrict__ x, const double *__restrict__ y,
@@ -2808,6 +3029,23 @@ int pair_grid_x(int N, int max_waves) {
   return (waves + 3) / 4;
 }
 
+// The FP64 table kernel with its table in LDS: whether a table of nsplin
+// points serves (it fits beside the kernel's 48 KB of staging, and is long
+// enough for the partial sums that reuse it), how many wavefronts share a
+// site, and the workgroups for a cap on wavefronts.
+bool pair_tab_lds_fits(int nsplin) {
+  return nsplin >= 512 && (size_t)nsplin * sizeof(double2) + 50 * 1024 <= FFT_LDS_MAX;
+}
+int pair_tab_wps(int N) {
+  int W = 1;
+  while (W < 4 && N * W * 2 <= 4096) W *= 2;
+  return W;
+}
+int pair_tab_grid_x(int N, int max_waves) {
+  const int sites = std::min(N, max_waves), W = pair_tab_wps(N);
+  return std::max(1, (sites * W + TAB_WAVES - 1) / TAB_WAVES);
+}
+
 // k_pair_mixed with the erfc term formed as TM says, with or without beads
 // and RESPA weights
 template <int B, int TM>
@@ -2826,7 +3064,13 @@ template <int B>
 void launch_pair_b(const PairArgs &a, int mode, bool full, dim3 grid, hipStream_t st) {
   const dim3 block(256);
   if (full) {
-    if (mode == 0) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pair_staged_tab<B>), grid, block, 0, st, a);
+    if (mode == 0 && a.wps > 0) {
+      const size_t lds = (size_t)a.nsplin * sizeof(double2);
+      const void *k = a.pimd ? (const void *)k_pair_tab_lds<B, true> : (const void *)k_pair_tab_lds<B, false>;
+      (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (a.pimd) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pair_tab_lds<B, true>), grid, dim3(64 * TAB_WAVES), lds, st, a);
+      else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pair_tab_lds<B, false>), grid, dim3(64 * TAB_WAVES), lds, st, a);
+    } else if (mode == 0) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pair_staged_tab<B>), grid, block, 0, st, a);
     else if (mode == 1) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pair_staged_dir<B>), grid, block, 0, st, a);
     else if (a.ftab && !a.respa) {
       const size_t lds = (size_t)a.nftab * CT_N * sizeof(float4);
