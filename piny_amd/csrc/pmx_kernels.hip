@@ -1581,7 +1581,7 @@ __device__ __forceinline__ double sqrt_normal(double x) {
 // in LDS).  The kernel then issues FP64 instructions: 109 a term, of which
 // the correctly rounded root, the interpolation's coefficients per function,
 // 64-bit addresses and the index's integer round trip were 40 (spline4_both,
-// sqrt_normal, byte offsets staged with the entries): TIMEUS us.
+// sqrt_normal, byte offsets staged with the entries): 540 us.
 //
 // a.wps wavefronts share a site, taking its row's chunks in turn, and add
 // their forces through LDS: with fewer sites than the 4096 wavefronts the
