@@ -3088,12 +3088,12 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
   if (int rc = pimd_force(c, flags)) return rc;
   const bool xmod_given = c->xmod_given;
   c->xmod_given = true;  // xmod is mode 1 of each drift from here on
-  const unsigned gN = blocks(N), gNP = blocks(NP);
+  const unsigned gN = blocks(N);
   int rc = PMX_OK;
   for (int step = 0; step < nsteps && !rc; step++) {
     hipLaunchKernelGGL(k_nhc_ckin, dim3(NHC_BLOCKS), dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_nhc_class, dim3(1), dim3(64), 0, c->st, a, NHC_BLOCKS);
-    hipLaunchKernelGGL(k_nhc_kick, dim3(gNP), dim3(256), 0, c->st, a, 0);
+    (void)launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);  // errors: the check below
+    (void)launch_nhc(a, NHC_KICK0, 0, c->st);
     hipLaunchKernelGGL(k_mode_drift, dim3(mode_blocks(N, P)), dim3(256), 0, c->st, a);
     if (c->nghost)
       hipLaunchKernelGGL(k_ghost_pos, dim3(blocks((size_t)c->nghost * P)), dim3(256), 0, c->st, c->nghost, P,
@@ -3103,9 +3103,9 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
       break;
     }
     if ((rc = pimd_force(c, flags))) break;
-    hipLaunchKernelGGL(k_nhc_kick, dim3(gNP), dim3(256), 0, c->st, a, 1);
+    (void)launch_nhc(a, NHC_KICK1, 0, c->st);
     hipLaunchKernelGGL(k_nhc_ckin, dim3(NHC_BLOCKS), dim3(256), 0, c->st, a);
-    hipLaunchKernelGGL(k_nhc_class, dim3(1), dim3(64), 0, c->st, a, NHC_BLOCKS);
+    (void)launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);
     hipLaunchKernelGGL(k_nhc_scale0, dim3(gN), dim3(256), 0, c->st, a);
   }
   c->xmod_given = xmod_given;

@@ -3151,19 +3151,24 @@ namespace pmx {
 
 // One Nose-Hoover chain of apply_NHC_par (md/int_NVT.c:144-330) over its
 // degrees of freedom, whose sum of m v^2 is kin; v, x are the chain's
-// velocities and positions (1-based, len of them).  Returns the factor the
-// degrees of freedom's velocities are scaled by.
-__device__ __forceinline__ double nhc_chain(const NhcArgs &a, const double *mass, const double *gkt, double *v,
-                                            double *x, double kin) {
+// velocities and positions (1-based, L of them).  Returns the factor the
+// degrees of freedom's velocities are scaled by.  The length is a template
+// parameter so that the links sit in registers: at a run-time length they
+// lived in per-lane memory, and the chain is one dependent sequence (84
+// exponentials at the usual 4 links, 4 x 3 steps).
+template <int L>
+__device__ __forceinline__ double nhc_chain(const NhcArgs &a, const double *mass, const double *gkt,
+                                            double (&v)[L + 1], double (&x)[L + 1], double kin) {
 #pragma clang fp contract(off)
-  const int L = a.len;
-  double f[8];
+  double f[L + 1];
   double sc = 1.0;
   f[1] = (kin - gkt[1]) / mass[1];
+#pragma unroll
   for (int ic = 1; ic <= L - 1; ic++) f[ic + 1] = (mass[ic] * v[ic] * v[ic] - gkt[ic + 1]) / mass[ic + 1];
   for (int ir = 1; ir <= a.nres; ir++) {
     for (int iy = 1; iy <= a.nyosh; iy++) {
       v[L] += f[L] * a.wdti4[iy];
+#pragma unroll
       for (int ic = 1; ic <= L - 1; ic++) {
         const double aa = exp(-a.wdti8[iy] * v[L + 1 - ic]);
         v[L - ic] = v[L - ic] * aa * aa + a.wdti4[iy] * f[L - ic] * aa;
@@ -3171,8 +3176,10 @@ __device__ __forceinline__ double nhc_chain(const NhcArgs &a, const double *mass
       const double aa = exp(-a.wdti2[iy] * v[1]);
       sc *= aa;
       kin *= aa * aa;
+#pragma unroll
       for (int ic = 1; ic <= L; ic++) x[ic] += v[ic] * a.wdti2[iy];
       f[1] = (kin - gkt[1]) / mass[1];
+#pragma unroll
       for (int ic = 1; ic <= L - 1; ic++) {
         const double a2 = exp(-a.wdti8[iy] * v[ic + 1]);
         v[ic] = v[ic] * a2 * a2 + a.wdti4[iy] * f[ic] * a2;
@@ -3203,70 +3210,97 @@ __global__ void __launch_bounds__(256) k_nhc_ckin(NhcArgs a) {
   if (threadIdx.x == 0) a.part[blockIdx.x] = red[0];
 }
 
-// The centroid chain (one thread): the kinetic sum in a fixed order, the
-// chain's evolution, and the scale factor in cls[2 len].
-__global__ void k_nhc_class(NhcArgs a, int G) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// The centroid chain (one wavefront): the kinetic sum over the partials in a
+// fixed order, the chain's evolution (every lane alike), and the scale factor
+// in cls[2 L].
+template <int L>
+__global__ void __launch_bounds__(64) k_nhc_class(NhcArgs a, int G) {
+  const int lane = threadIdx.x;
   double kin = 0.0;
-  for (int g = 0; g < G; g++) kin += a.part[g];
-  const int L = a.len;
-  double v[8], x[8];
+  for (int g = lane; g < G; g += 64) kin += a.part[g];
+  kin = wave_sum_mod(kin, 1);
+  double v[L + 1], x[L + 1];
+#pragma unroll
   for (int j = 1; j <= L; j++) {
     v[j] = a.cls[j - 1];
     x[j] = a.cls[L + j - 1];
   }
-  const double sc = nhc_chain(a, a.cmass, a.cgkt, v, x, kin);
-  for (int j = 1; j <= L; j++) {
-    a.cls[j - 1] = v[j];
-    a.cls[L + j - 1] = x[j];
+  const double sc = nhc_chain<L>(a, a.cmass, a.cgkt, v, x, kin);
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 1; j <= L; j++) {
+      a.cls[j - 1] = v[j];
+      a.cls[L + j - 1] = x[j];
+    }
+    a.cls[2 * L] = sc;
   }
-  a.cls[2 * L] = sc;
 }
 
-// One thread per (site, mode): phase 0 is the first half step (chains, then
-// the kick: int_0_to_dt2_nvt_pimd sections 1-2), phase 1 the second (the
-// kick, then the chains of modes 2..P; the centroid mode is scaled by
-// k_nhc_scale0 once its chain has run).  The centroid mode's velocities are
-// scaled by the centroid chain's factor in phase 0; every other mode's
-// degree of freedom runs its own chain with the mode mass.
+// One thread per (direction, site, mode): phase 0 is the first half step
+// (chains, then the kick: int_0_to_dt2_nvt_pimd sections 1-2), phase 1 the
+// second (the kick, then the chains of modes 2..P; the centroid mode is
+// scaled by k_nhc_scale0 once its chain has run).  The centroid mode's
+// velocities are scaled by the centroid chain's factor in phase 0; every
+// other mode's degree of freedom runs its own chain with the mode mass.
+// Latency bound: 343 SPC/Fw at P = 16 are 774 wavefronts, three a CU.  One
+// thread a (site, mode) with the three chains in turn and their links in
+// per-lane memory took 59 us there, this 10 us.
+template <int L>
 __global__ void __launch_bounds__(256) k_nhc_kick(NhcArgs a, int phase) {
 #pragma clang fp contract(off)
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x, NP = (size_t)a.N * a.P;
-  if (t >= NP) return;
+  const size_t u = (size_t)blockIdx.x * blockDim.x + threadIdx.x, NP = (size_t)a.N * a.P;
+  if (u >= 3 * NP) return;
+  const int d = (int)(u / NP);
+  const size_t t = u - (size_t)d * NP;
   const int i = (int)(t / a.P), m = (int)(t - (size_t)i * a.P);
   const double mm = a.mass[i] * a.mfac[m];
-  double *vv[3] = {a.vx, a.vy, a.vz};
-  const double *ff[3] = {a.fx, a.fy, a.fz};
+  double *vv = d == 0 ? a.vx : d == 1 ? a.vy : a.vz;
+  const double *ff = d == 0 ? a.fx : d == 1 ? a.fy : a.fz;
   const bool real = a.ghost[i] == 0;
-  auto chains = [&]() {
-    if (!real) return;
-    if (m == 0) {
-      if (phase == 0) {
-        const double sc = a.cls[2 * a.len];
-        for (int d = 0; d < 3; d++) vv[d][t] *= sc;
-      }
-      return;
+  double vd = vv[t];
+  const double kick = ff[t] * a.dt2 / mm;
+  if (phase == 1) vd += kick;
+  if (real && m == 0 && phase == 0) vd *= a.cls[2 * L];
+  if (real && m != 0) {
+    double v[L + 1], x[L + 1];
+#pragma unroll
+    for (int j = 1; j <= L; j++) {
+      const size_t o = ((size_t)((j - 1) * 3 + d)) * NP + t;
+      v[j] = a.vnhc[o];
+      x[j] = a.xnhc[o];
     }
-    for (int d = 0; d < 3; d++) {
-      double v[8], x[8];
-      for (int j = 1; j <= a.len; j++) {
-        const size_t o = ((size_t)((j - 1) * 3 + d)) * NP + t;
-        v[j] = a.vnhc[o];
-        x[j] = a.xnhc[o];
-      }
-      const double vd = vv[d][t];
-      const double sk = nhc_chain(a, a.bmass, a.bgkt, v, x, mm * vd * vd);
-      vv[d][t] = vd * sk;
-      for (int j = 1; j <= a.len; j++) {
-        const size_t o = ((size_t)((j - 1) * 3 + d)) * NP + t;
-        a.vnhc[o] = v[j];
-        a.xnhc[o] = x[j];
-      }
+    vd *= nhc_chain<L>(a, a.bmass, a.bgkt, v, x, mm * vd * vd);
+#pragma unroll
+    for (int j = 1; j <= L; j++) {
+      const size_t o = ((size_t)((j - 1) * 3 + d)) * NP + t;
+      a.vnhc[o] = v[j];
+      a.xnhc[o] = x[j];
     }
-  };
-  if (phase == 0) chains();
-  for (int d = 0; d < 3; d++) vv[d][t] += ff[d][t] * a.dt2 / mm;
-  if (phase == 1) chains();
+  }
+  if (phase == 0) vd += kick;
+  vv[t] = vd;
+}
+
+template <int L>
+static void launch_nhc_len(const NhcArgs &a, int what, int G, hipStream_t st) {
+  const size_t n = (size_t)3 * a.N * a.P;
+  if (what == NHC_CLASS) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_nhc_class<L>), dim3(1), dim3(64), 0, st, a, G);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_nhc_kick<L>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a,
+                       what == NHC_KICK1 ? 1 : 0);
+}
+
+hipError_t launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st) {
+  switch (a.len) {
+    case 1: launch_nhc_len<1>(a, what, G, st); break;
+    case 2: launch_nhc_len<2>(a, what, G, st); break;
+    case 3: launch_nhc_len<3>(a, what, G, st); break;
+    case 4: launch_nhc_len<4>(a, what, G, st); break;
+    case 5: launch_nhc_len<5>(a, what, G, st); break;
+    case 6: launch_nhc_len<6>(a, what, G, st); break;
+    default: launch_nhc_len<7>(a, what, G, st); break;  // the length is checked to be 1..7
+  }
+  return hipGetLastError();
 }
 
 // the centroid mode's velocities scaled by its chain's factor (phase 1)
@@ -3426,14 +3460,16 @@ __global__ void __launch_bounds__(256) k_pimd_energy(NhcArgs a) {
   }
 }
 
-// out[0] kinetic, out[1] chain energy with the centroid chain (one thread)
-__global__ void k_pimd_energy_sum(NhcArgs a, int G, double *out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// out[0] kinetic, out[1] chain energy with the centroid chain (one wavefront)
+__global__ void __launch_bounds__(64) k_pimd_energy_sum(NhcArgs a, int G, double *out) {
   double ke = 0.0, en = 0.0;
-  for (int g = 0; g < G; g++) {
+  for (int g = threadIdx.x; g < G; g += 64) {
     ke += a.part[2 * g];
     en += a.part[2 * g + 1];
   }
+  ke = wave_sum_mod(ke, 1);
+  en = wave_sum_mod(en, 1);
+  if (threadIdx.x != 0) return;
   const int L = a.len;
   for (int j = 1; j <= L; j++) en += 0.5 * a.cmass[j] * a.cls[j - 1] * a.cls[j - 1] + a.cgkt[j] * a.cls[L + j - 1];
   out[0] = ke;

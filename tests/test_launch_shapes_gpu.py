@@ -74,3 +74,28 @@ def test_pair_table_in_lds(nmol, P, nsplin):
     c = w.small_config(w.SPC_FW, nmol=nmol, P=P, seed=nmol)
     c.system.settings.nsplin = nsplin
     check(c)
+
+
+# Nose-Hoover chains: every length is a kernel of its own; the state against
+# the oracle's integrator
+@pytest.mark.parametrize("len_nhc", [1, 2, 3, 4, 5, 6, 7])
+def test_chain_lengths(len_nhc):
+    from piny_amd.engine import Engine
+    c = w.small_config(w.Q_TIP4P_F, nmol=27, P=4, seed=9)
+    par = abi.nhc_params(len_nhc=len_nhc)
+    rng = np.random.default_rng(len_nhc)
+    v = rng.normal(size=(3, c.x.size)) * 1e-4
+    v.reshape(3, 4, -1)[:, :, c.system.ghost_atom] = 0.0
+    eng = Engine(c.system, c.x, c.y, c.z)
+    eng.set_positions(c.x, c.y, c.z)
+    eng.set_velocities(*v)
+    _, ec = eng.pimd_nvt(3, par)
+    vel, x, chains = eng.velocities(), eng.positions(), eng.nhc_state()
+    o = Oracle(c.system, c.x, c.y, c.z)
+    v0 = v.reshape(3, 4, -1).transpose(1, 2, 0)
+    xo, vo, st, _, eco = o.pimd_nvt(3, c.x, c.y, c.z, v0, params=par)
+    assert np.abs(x - xo).max() < 1e-9 * np.abs(xo).max()
+    assert np.abs(vel - vo).max() < 1e-9 * np.abs(vo).max()
+    assert np.abs(chains - st).max() < 1e-9 * np.abs(st).max()
+    assert abs(ec[3] - eco[3]) < 1e-9 * np.abs(eco).max()
+    eng.close()
