@@ -82,7 +82,7 @@ struct pmx_ctx {
   std::vector<float4> ft_host;  // the whole switched pair functions [nftab][CT_N]
   bool full_list = true;   // force list with both directions (no atomics)
   int cap = 0, *jfull = nullptr, *jforce = nullptr, *nfull = nullptr, *nforce = nullptr, *overflow = nullptr;
-  int *jsplit = nullptr;  // the force list's second buffer (rows split by the cutoff)
+  int *jsplit = nullptr;  // the force list's rows as built, before they are split by the cutoff into jforce
   // link cells of the list build
   int *site_cell = nullptr, *site_pos = nullptr, *cell_cnt = nullptr, *cell_start = nullptr, *cell_sites = nullptr;
   bool list_cells = false;  // the last build used link cells
@@ -91,6 +91,8 @@ struct pmx_ctx {
   PairTypes pt_build{};     // cut+skin at the last build
   double4 *cell_p = nullptr, *cell_m = nullptr;  // sites in cell order (link-cell build)
   int *cell_i = nullptr;
+  float4 *cell_f = nullptr;
+  int *ov_pin = nullptr;  // pinned: the longest row and the pair count of a build
   int *b1 = nullptr, *b2 = nullptr, *btyp = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr,
       *atyp = nullptr, *e1 = nullptr, *e2 = nullptr;
   double *bc = nullptr, *beq = nullptr, *ac = nullptr, *as = nullptr;
@@ -158,7 +160,6 @@ struct pmx_ctx {
   // scan, 2 link cells)
   int tile_cap[3] = {16, 16, 8};
   int pair_waves = 4096;
-  int list_waves = 8;         // wavefronts per cell of the link-cell list build (4: 448 us, 8: 322 us, 16: slower)
   int list_mode = 0;
   hipEvent_t ready = nullptr;  // list stage done (batched calls)
   // PME on a second stream, concurrent with the pair kernel (the pair
@@ -1012,6 +1013,7 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
   TRY(dalloc(c, &c->cell_p, N));
   TRY(dalloc(c, &c->cell_m, N));
   TRY(dalloc(c, &c->cell_i, N));
+  TRY(dalloc(c, &c->cell_f, N));
   TRY(dalloc(c, &c->xm0, N));
   TRY(dalloc(c, &c->ym0, N));
   TRY(dalloc(c, &c->zm0, N));
@@ -1164,6 +1166,7 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
   TRY(dalloc(c, &c->acc, (size_t)P * ACC_NUM + 1));
   c->ake = c->acc + (size_t)P * ACC_NUM;
   c->acc_h.assign((size_t)P * ACC_NUM, 0.0);
+  HIPCHK(hipHostMalloc((void **)&c->ov_pin, 4 * sizeof(int), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void **)&c->mx_pin, 2 * LIST_CHECK_BLOCKS * sizeof(double), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void **)&c->acc_pin, ((size_t)P * ACC_NUM + 1) * sizeof(double), hipHostMallocDefault));
   TRY(upload(c, &c->prekf, s.prekf.data(), N));
@@ -1201,9 +1204,12 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
 // so that the (2H + 1)^3 cells around a site's cell hold every site with an
 // image inside the list radius, each once.  H = 2 when the box allows it
 // (a 5^3 stencil of half-width cells: about 3.7 candidates per list pair),
-// else H = 1 (27 cells); 0 when the box is too small for either, or the
-// plain scan is asked for (PMX_LIST=brute, or the autotuner's choice), and
-// the ascending O(N^2) scan is used.
+// else H = 1 (27 cells); 0, which tests every site, when the box is too small
+// for either or the cells spare a site fewer than 6000 candidates: their
+// sorting is five launches more (list stage of a rebuild without and with
+// cells: 144 and 155 us at 8000 sites, 5100 candidates spared; 226 and 200 us
+// at 12000, 9900 spared; 305 and 216 us at 16384).  PMX_LIST=brute|cells and
+// the autotuner choose otherwise.
 int choose_cells(const pmx_ctx *c, int nc[3]) {
   const char *env = getenv("PMX_LIST");  // tuning override: "brute" or "cells"
   if ((env && strcmp(env, "brute") == 0) || c->list_mode == 1) return 0;
@@ -1219,7 +1225,9 @@ int choose_cells(const pmx_ctx *c, int nc[3]) {
       ok = ok && nc[d] >= 2 * H + 1;
       ncell *= (size_t)std::max(nc[d], 1);
     }
-    if (ok && ncell <= (size_t)MAX_LIST_CELLS) return H;
+    if (!ok || ncell > (size_t)MAX_LIST_CELLS) continue;
+    const double spared = (double)c->s.N * (1.0 - (2 * H + 1) * (2 * H + 1) * (2 * H + 1) / (double)ncell);
+    return env || c->list_mode == 2 || spared >= 6000.0 ? H : 0;
   }
   return 0;
 }
@@ -1245,6 +1253,7 @@ ListArgs list_args(pmx_ctx *c) {
   a.cell = c->cell;
   a.full = c->full_list ? 1 : 0;
   a.jfull = c->jfull;
+  a.jrow = c->jsplit;
   a.jforce = c->jforce;
   a.nfull = c->nfull;
   a.nforce = c->nforce;
@@ -1257,6 +1266,7 @@ ListArgs list_args(pmx_ctx *c) {
   a.cell_p = c->cell_p;
   a.cell_m = c->cell_m;
   a.cell_i = c->cell_i;
+  a.cell_f = c->cell_f;
   return a;
 }
 
@@ -1272,8 +1282,14 @@ int build_list(pmx_ctx *c) {
     const int H = cells_failed ? 0 : choose_cells(c, nc);
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->st, c->overflow, 0, (size_t)4);
     ListArgs a = list_args(c);
-    a.use_cells = 0;
     for (int d = 0; d < 3; d++) a.nc[d] = nc[d];
+    // the FP32 test's radius: the largest cut+skin, with room for fractions
+    // rounded to 24 bits; no test in cells that are not orthorhombic
+    double rl = 0.0, hmax = 0.0;
+    for (int t = 0; t < s.npair; t++) rl = std::max(rl, sqrt(c->pt.cutskin2[t]));
+    for (int d = 0; d < 3; d++) hmax = std::max(hmax, fabs(c->cell.h[4 * d]));
+    rl = (rl + 1e-6 * hmax) * (1.0 + 1e-5);
+    a.lim2 = c->cell.cubic ? (float)(rl * rl) : HUGE_VALF;
     if (H > 0) {
       const int ncell = nc[0] * nc[1] * nc[2];
       hipLaunchKernelGGL(k_fill_int, dim3(blocks(ncell)), dim3(256), 0, c->st, c->cell_cnt, 0, (size_t)ncell);
@@ -1281,33 +1297,28 @@ int build_list(pmx_ctx *c) {
       hipLaunchKernelGGL(k_cell_scan, dim3(1), dim3(256), 0, c->st, ncell, c->cell_cnt, c->cell_start);
       hipLaunchKernelGGL(k_cell_scatter, dim3(blocks(s.N)), dim3(256), 0, c->st, a);
       hipLaunchKernelGGL(k_cell_order, dim3(ncell), dim3(256), 0, c->st, a);
-      HIPCHK(hipGetLastError());
-      HIPCHK(launch_list_cells(a, H, ncell, c->list_waves, c->st));
     } else {
-      hipLaunchKernelGGL(k_list_build, dim3(blocks((size_t)s.N * 64)), dim3(256), 0, c->st, a);
-      HIPCHK(hipGetLastError());
+      hipLaunchKernelGGL(k_list_records, dim3(blocks(s.N)), dim3(256), 0, c->st, a);
     }
-    int ov[4];
-    HIPCHK(hipMemcpyAsync(ov, c->overflow, sizeof ov, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipGetLastError());
+    HIPCHK(launch_list_rows(a, H, c->st));
+    hipLaunchKernelGGL(k_list_counts, dim3(1), dim3(1024), 0, c->st, a);
+    const int *ov = c->ov_pin;
+    HIPCHK(hipMemcpyAsync(c->ov_pin, c->overflow, 4 * sizeof(int), hipMemcpyDeviceToHost, c->st));
+    // behind the readback: the rows with the pairs inside the cutoff first,
+    // and the state the checks and the reference list go back to
+    hipLaunchKernelGGL(k_split_rows, dim3(blocks((size_t)s.N * 64)), dim3(256), 0, c->st, a);
+    hipLaunchKernelGGL(k_list_keep, dim3(blocks(s.N)), dim3(256), 0, c->st, s.N, c->b0x, c->b0y, c->b0z, c->xm, c->ym,
+                       c->zm, c->x0, c->y0, c->z0, c->xm0, c->ym0, c->zm0);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->st));
-    if (ov[2]) {  // a cell too full for the cell kernels: the plain scan
+    if (ov[2]) {  // a cell too full to be ordered: no cells
       cells_failed = true;
       continue;
     }
     if (ov[0] == 0) {
-      // force-list rows: pairs inside the cutoff first
-      hipLaunchKernelGGL(k_split_rows, dim3(blocks((size_t)s.N * 64)), dim3(256), 0, c->st, a, c->jsplit);
-      HIPCHK(hipGetLastError());
-      // copied back rather than swapped: captured force sequences keep
-      // pointing at jforce
-      HIPCHK(hipMemcpyAsync(c->jforce, c->jsplit, (size_t)s.N * c->cap * sizeof(int), hipMemcpyDeviceToDevice,
-                            c->st));
-      // the state the reference list is built from on demand
-      HIPCHK(hipMemcpyAsync(c->xm0, c->xm, s.N * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-      HIPCHK(hipMemcpyAsync(c->ym0, c->ym, s.N * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-      HIPCHK(hipMemcpyAsync(c->zm0, c->zm, s.N * sizeof(double), hipMemcpyDeviceToDevice, c->st));
       c->pt_build = c->pt;
-      c->ref_valid = (H == 0);  // the plain scan also wrote the reference's rows
+      c->ref_valid = false;
       c->list_cells = H > 0;
       c->nver = ov[1];
       if (c->clu_ok && c->clu_enabled) {
@@ -1341,6 +1352,7 @@ int build_ref_list(pmx_ctx *c) {
   a.ref_only = 1;
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->st, c->overflow, 0, (size_t)4);
   hipLaunchKernelGGL(k_list_build, dim3(blocks((size_t)c->s.N * 64)), dim3(256), 0, c->st, a);
+  hipLaunchKernelGGL(k_list_counts, dim3(1), dim3(1024), 0, c->st, a);
   HIPCHK(hipGetLastError());
   int ov[4];
   HIPCHK(hipMemcpyAsync(ov, c->overflow, sizeof ov, hipMemcpyDeviceToHost, c->st));
@@ -1506,11 +1518,8 @@ int list_stage_finish(pmx_ctx *c, unsigned flags, pmx_energies *out) {
   }
   if (rebuild) {
     if (P > 1) c->spread = spread_now;
-    HIPCHK(hipMemcpyAsync(c->x0, c->b0x, N * sizeof(double), hipMemcpyDeviceToDevice, st));
-    HIPCHK(hipMemcpyAsync(c->y0, c->b0y, N * sizeof(double), hipMemcpyDeviceToDevice, st));
-    HIPCHK(hipMemcpyAsync(c->z0, c->b0z, N * sizeof(double), hipMemcpyDeviceToDevice, st));
-    int rc = build_list(c);
-    if (rc) return rc;
+    c->have_list = false;  // a build that fails leaves none
+    if (int rc = build_list(c)) return rc;
     c->have_list = true;
   }
   out->list_rebuilt = rebuild;
@@ -2165,8 +2174,6 @@ pmx_ctx *pmx_create(const pmx_system *sys, const pmx_params *par, const double *
   if (const char *env = getenv("PMX_CLUSTER")) c->clu_enabled = atoi(env) == 1;
   if (const char *env = getenv("PMX_PAIR_WAVES"))  // tuning override: wavefronts of the pair kernels
     c->pair_waves = std::max(64, std::min(PAIR_MAX_WAVES, atoi(env)));
-  if (const char *env = getenv("PMX_LIST_WAVES"))  // tuning override: wavefronts per cell of the list build
-    c->list_waves = atoi(env) >= 16 ? 16 : (atoi(env) >= 8 ? 8 : 4);
   if (const char *env = getenv("PMX_PME_TILE"))  // tuning override "Ta,Tb,Tc" (upper bounds)
     sscanf(env, "%d,%d,%d", &c->tile_cap[0], &c->tile_cap[1], &c->tile_cap[2]);
   if (build_device(c, sys) != PMX_OK) {
@@ -2187,6 +2194,7 @@ void pmx_destroy(pmx_ctx *c) {
   if (c->st) (void)hipStreamSynchronize(c->st);
   if (c->sk) (void)hipStreamSynchronize(c->sk);
   for (void *p : c->allocs) (void)hipFree(p);
+  if (c->ov_pin) (void)hipHostFree(c->ov_pin);
   if (c->mx_pin) (void)hipHostFree(c->mx_pin);
   if (c->acc_pin) (void)hipHostFree(c->acc_pin);
   for (auto &e : c->ev)

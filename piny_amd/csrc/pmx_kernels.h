@@ -10,15 +10,18 @@ namespace pmx {
 struct ListArgs {
   int N, cap, pimd;
   int full;  // 1: jforce holds every interacting j != i (both directions)
-  int ref_only;  // k_list_build: write the reference's half list only (jfull, nfull)
-  // link cells (when use_cells): nc[3] cells per axis of fractional space,
-  // sites of cell k at cell_sites[cell_start[k] .. + cell_cnt[k]]
-  int use_cells, nc[3];
+  int ref_only;  // k_list_counts: only the reference's half list was built
+  // link cells: nc[3] cells per axis of fractional space, sites of cell k at
+  // cell_sites[cell_start[k] .. + cell_cnt[k]]
+  int nc[3];
   int *site_cell, *site_pos, *cell_cnt, *cell_start, *cell_sites;
-  // k_list_cells: the sites in cell order, (bead-1 x, y, z, q) and
-  // (xmod x, y, z, type as a double), and the site index
+  // k_list_rows: the sites in cell order (or as they are), (bead-1 x, y, z,
+  // q), (xmod x, y, z, type as a double), bead 1's fractions of the cell in
+  // [0, 1), and the site index; lim2 the square of the FP32 test's radius
   double4 *cell_p, *cell_m;
+  float4 *cell_f;
   int *cell_i;
+  float lim2;
   const double *bx, *by, *bz;  // bead-1 positions [N]
   const double *xm, *ym, *zm;  // xmod [N]
   const int *type;
@@ -26,7 +29,7 @@ struct ListArgs {
   const int *ex_off, *ex_num, *ex_j;  // exclusions (both directions when full)
   PairTypes pt;
   Cell cell;
-  int *jfull, *jforce;  // ELL rows of width cap
+  int *jfull, *jrow, *jforce;  // ELL rows of width cap: reference list, force list as built, and split
   int *nfull, *nforce;
   int *overflow;
 };
@@ -375,19 +378,21 @@ __global__ void k_cell_count(ListArgs a);
 __global__ void k_cell_scan(int ncell, const int *cnt, int *start);
 __global__ void k_cell_scatter(ListArgs a);
 constexpr int CELL_SORT_MAX = 1024;  // sites of one cell k_cell_order sorts in LDS
-constexpr int CELL_ROWS_MAX = 512;   // sites of one cell whose rows one k_list_cells workgroup keeps
-constexpr int CELL_TILE = 320;       // candidate sites one k_list_cells workgroup stages in LDS at a time
 constexpr int SPLIT_CHUNKS = 32;     // 64-entry chunks of a row whose inside flags k_split_rows keeps
 __global__ void k_cell_order(ListArgs a);
-hipError_t launch_list_cells(const ListArgs &a, int halfwidth, int ncell, int nw, hipStream_t st);
-__global__ void k_sort_rows(int cap, int n2, const int *nfull, const int *nforce, int *jfull, int *jforce);
+__global__ void k_list_records(ListArgs a);
+hipError_t launch_list_rows(const ListArgs &a, int halfwidth, hipStream_t st);
+__global__ void k_list_counts(ListArgs a);
+__global__ void k_list_keep(int N, const double *b0, const double *b1, const double *b2, const double *m0,
+                            const double *m1, const double *m2, double *x0, double *y0, double *z0, double *xm0,
+                            double *ym0, double *zm0);
 __global__ void k_pme_bin(PmeArgs a);
 __global__ void k_pme_scan(PmeArgs a);
 __global__ void k_pme_scatter(PmeArgs a);
 __global__ void k_fill_int(int *p, int v, size_t n);
 __global__ void k_fill_double(double *p, double v, size_t n);
 __global__ void k_reduce_partials(RedArgs a);
-__global__ void k_split_rows(ListArgs a, int *out);
+__global__ void k_split_rows(ListArgs a);
 __global__ void k_ecor_phi(IntraArgs a);
 __global__ void k_bond_moments(IntraArgs a);
 __global__ void k_bend_moments(IntraArgs a);

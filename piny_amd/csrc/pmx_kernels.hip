@@ -370,11 +370,10 @@ __global__ void __launch_bounds__(256) k_list_check(int N, int P, const double *
 
 // ---------------------------------------------------------------------------
 // Verlet list: nolst_ver_gen + verlist_create (verlist_control.c:134-441,
-// verlist_create.c:223-503).  One wavefront per site i scans j in ascending
-// chunks of 64; a ballot keeps the reference's order, so each per-site
-// segment comes out sorted.  Two lists are written in ELL form (row i at
-// i*cap): the reference's half list (j < i, r^2 < cutskin^2) and the list the
-// force kernel walks, which keeps only pairs that can interact (LJ table
+// verlist_create.c:223-503).  Two lists in ELL form (row i at i*cap): the
+// reference's half list (j < i ascending, r^2 < cutskin^2; k_list_build, one
+// wavefront per site, on demand) and the list the force kernels walk
+// (k_list_rows), which keeps only pairs that can interact (LJ table
 // non-null or q_i q_j != 0) and, when full is set, holds both directions
 // (every j != i).  The minimum image is odd in the separation, so the full
 // list is exactly the half list and its transpose.  No FMA contraction: the
@@ -436,81 +435,37 @@ __global__ void __launch_bounds__(256) k_list_build(ListArgs a) {
     zmi = a.zm[i];
   }
   const int ti = a.type[i];
-  const double qi = a.q[i];
   const int eo = a.ex_off[i], en = a.ex_num[i];
-  int nfull = 0, nforce = 0;
+  int nfull = 0;
   int *rowf = a.jfull + (size_t)i * a.cap;
-  int *rowi = a.jforce + (size_t)i * a.cap;
-  // candidates: every j (ascending, so rows come out sorted) or the sites of
-  // the 27 link cells around i's cell (rows sorted afterwards by k_sort_rows)
-  const int jend = a.full ? a.N : i;
-  const int ncand_cells = a.use_cells ? 27 : 1;
-  int ci[3] = {0, 0, 0};
-  if (a.use_cells) {
-    const int c0 = a.site_cell[i];
-    ci[0] = c0 % a.nc[0];
-    ci[1] = (c0 / a.nc[0]) % a.nc[1];
-    ci[2] = c0 / (a.nc[0] * a.nc[1]);
-  }
-  for (int cc = 0; cc < ncand_cells; cc++) {
-    int base = 0, count = jend;
-    const int *sites = nullptr;
-    if (a.use_cells) {
-      int n3[3];
-      const int off[3] = {cc % 3 - 1, (cc / 3) % 3 - 1, cc / 9 - 1};
-#pragma unroll
-      for (int d = 0; d < 3; d++) n3[d] = (ci[d] + off[d] + a.nc[d]) % a.nc[d];
-      const int cell = (n3[2] * a.nc[1] + n3[1]) * a.nc[0] + n3[0];
-      base = a.cell_start[cell];
-      count = a.cell_cnt[cell];
-      sites = a.cell_sites;
-    }
-    for (int j0 = 0; j0 < count; j0 += 64) {
-      const int jj = j0 + lane;
-      const int j = (jj < count) ? (sites ? sites[base + jj] : jj) : a.N;
-      bool keep = false, inter = false;
-      int t = 0;
-      if (j < a.N && (a.full || j < i) && j != i) {
-        bool excl = false;
-        for (int k = 0; k < en; k++) excl |= (a.ex_j[eo + k] == j);
-        if (!excl) {
-          double dx, dy, dz;
-          double xmj = 0.0, ymj = 0.0, zmj = 0.0;
-          if (a.pimd) {
-            xmj = a.xm[j];
-            ymj = a.ym[j];
-            zmj = a.zm[j];
-          }
-          const double r2 = min_image_sep(a.cell, a.pimd, xi, yi, zi, a.bx[j], a.by[j], a.bz[j], xmi, ymi, zmi, xmj,
-                                          ymj, zmj, dx, dy, dz);
-          t = pair_index(a.pt.ntype, ti, a.type[j]);
-          const bool in = r2 < a.pt.cutskin2[t];
-          keep = in && j < i;
-          inter = in && (a.pt.lj[t] || (qi * a.q[j] != 0.0));
+  for (int j0 = 0; j0 < i; j0 += 64) {
+    const int j = j0 + lane;
+    bool keep = false;
+    if (j < i) {
+      bool excl = false;
+      for (int k = 0; k < en; k++) excl |= (a.ex_j[eo + k] == j);
+      if (!excl) {
+        double dx, dy, dz;
+        double xmj = 0.0, ymj = 0.0, zmj = 0.0;
+        if (a.pimd) {
+          xmj = a.xm[j];
+          ymj = a.ym[j];
+          zmj = a.zm[j];
         }
+        const double r2 = min_image_sep(a.cell, a.pimd, xi, yi, zi, a.bx[j], a.by[j], a.bz[j], xmi, ymi, zmi, xmj,
+                                        ymj, zmj, dx, dy, dz);
+        keep = r2 < a.pt.cutskin2[pair_index(a.pt.ntype, ti, a.type[j])];
       }
-      if (a.ref_only) inter = false;
-      const unsigned long long mk = __ballot(keep), mi = __ballot(inter);
-      const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-      if (keep) {
-        const int p = nfull + __popcll(mk & below);
-        if (p < a.cap) rowf[p] = j;
-      }
-      if (inter) {
-        const int p = nforce + __popcll(mi & below);
-        if (p < a.cap) rowi[p] = j | (t << ENTRY_SHIFT);
-      }
-      nfull += __popcll(mk);
-      nforce += __popcll(mi);
     }
+    const unsigned long long mk = __ballot(keep);
+    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    if (keep) {
+      const int p = nfull + __popcll(mk & below);
+      if (p < a.cap) rowf[p] = j;
+    }
+    nfull += __popcll(mk);
   }
-  if (lane == 0) {
-    a.nfull[i] = nfull;
-    if (!a.ref_only) a.nforce[i] = nforce;
-    const int mx = nfull > nforce ? nfull : nforce;
-    if (mx > a.cap) atomicMax(a.overflow, mx);
-    atomicAdd(a.overflow + 1, nfull);  // pair count of the reference list
-  }
+  if (lane == 0) a.nfull[i] = nfull;
 }
 
 // Link cells (make_lnk_lst.c:37-355 bins atoms into cells of fractional
@@ -565,6 +520,23 @@ __global__ void __launch_bounds__(256) k_cell_scatter(ListArgs a) {
   a.cell_sites[a.cell_start[a.site_cell[i]] + a.site_pos[i]] = i;
 }
 
+// The records of site v at place d of the candidate order.
+__device__ __forceinline__ void list_record(const ListArgs &a, int d, int v) {
+  const double x = a.bx[v], y = a.by[v], z = a.bz[v];
+  a.cell_i[d] = v;
+  a.cell_p[d] = make_double4(x, y, z, a.q[v]);
+  a.cell_m[d] = a.pimd ? make_double4(a.xm[v], a.ym[v], a.zm[v], (double)a.type[v])
+                       : make_double4(0.0, 0.0, 0.0, (double)a.type[v]);
+  const Cell &c = a.cell;
+  double f[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    f[k] = x * c.hi[k] + y * c.hi[k + 3] + z * c.hi[k + 6];
+    f[k] -= floor(f[k]);
+  }
+  a.cell_f[d] = make_float4((float)f[0], (float)f[1], (float)f[2], 0.0f);
+}
+
 // Puts each cell's sites in ascending index order (one workgroup per cell;
 // the counting sort's atomics leave them in arbitrary order), so that the
 // cell order, and the force-list order that follows it, is the same on
@@ -586,188 +558,14 @@ __global__ void __launch_bounds__(256) k_cell_order(ListArgs a) {
     for (int m = 0; m < n; m++) rank += ids[m] < v;
     const int d = o + rank;
     a.cell_sites[d] = v;
-    a.cell_i[d] = v;
-    a.cell_p[d] = make_double4(a.bx[v], a.by[v], a.bz[v], a.q[v]);
-    a.cell_m[d] = a.pimd ? make_double4(a.xm[v], a.ym[v], a.zm[v], (double)a.type[v])
-                         : make_double4(0.0, 0.0, 0.0, (double)a.type[v]);
+    list_record(a, d, v);
   }
 }
 
-// Verlet list by link cells (make_lnk_lst.c:37-355, lnk_ver_gen_pad in
-// verlist_control.c:1738-2254): cells of fractional space at least
-// r_list / H wide, at least 2H + 1 per axis, so that the (2H + 1)^3 cells
-// around a site's cell hold every site within the list radius, each once.
-// One workgroup per cell.  For each row of 2H + 1 cells along a of the
-// stencil (contiguous in cell order, up to the wrap) the workgroup stages
-// the sites' records in LDS (CELL_TILE at a time); each wavefront takes
-// the cell's own sites in turn and tests 64 staged candidates per step:
-// the reference's image separation and cut+skin test (min_image_sep, the
-// same bits as the plain scan), then, for pairs inside, the exclusion
-// list.  A ballot appends the interacting pairs to the site's force-list
-// row (every j != i, or j < i for the half list), in stencil order; the
-// reference's half-list pairs (j < i, every type pair) are only counted
-// (nver).  Rows of the cell's sites are counted in LDS across the tiles.
-template <int H, int NW>
-__global__ void __launch_bounds__(64 * NW) k_list_cells(ListArgs a) {
-#pragma clang fp contract(off)
-  __shared__ double4 tp[CELL_TILE], tm[CELL_TILE];
-  __shared__ int ti[CELL_TILE];
-  __shared__ int rowf[CELL_ROWS_MAX], rowr[CELL_ROWS_MAX];
-  __shared__ int red[NW];
-  constexpr int W = 2 * H + 1;
-  const int c = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int ni = a.cell_cnt[c], oi = a.cell_start[c];
-  if (ni > CELL_ROWS_MAX) {  // uniform over the workgroup
-    if (threadIdx.x == 0) a.overflow[2] = 1;
-    return;
-  }
-  for (int k = threadIdx.x; k < ni; k += blockDim.x) {
-    rowf[k] = 0;
-    rowr[k] = 0;
-  }
-  const int ca = c % a.nc[0], cb = (c / a.nc[0]) % a.nc[1], cc = c / (a.nc[0] * a.nc[1]);
-  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int st = 0; st < W * W; st++) {
-    const int nb = (cb + st % W - H + a.nc[1]) % a.nc[1], nz = (cc + st / W - H + a.nc[2]) % a.nc[2];
-    // the row's cells: their starts and the running count before each
-    int rs[W], pre[W + 1];
-    pre[0] = 0;
-#pragma unroll
-    for (int d = 0; d < W; d++) {
-      const int na = (ca + d - H + a.nc[0]) % a.nc[0];
-      const int cell = (nz * a.nc[1] + nb) * a.nc[0] + na;
-      rs[d] = a.cell_start[cell];
-      pre[d + 1] = pre[d] + a.cell_cnt[cell];
-    }
-    const int tot = pre[W];
-    for (int t0 = 0; t0 < tot; t0 += CELL_TILE) {
-      const int nt = min(CELL_TILE, tot - t0);
-      __syncthreads();  // the previous tile's readers are done (and the row counters are cleared)
-      for (int e = threadIdx.x; e < nt; e += blockDim.x) {
-        const int g = t0 + e;
-        int src = 0;
-#pragma unroll
-        for (int d = 0; d < W; d++)
-          if (g >= pre[d] && g < pre[d + 1]) src = rs[d] + (g - pre[d]);
-        tp[e] = a.cell_p[src];
-        tm[e] = a.cell_m[src];
-        ti[e] = a.cell_i[src];
-      }
-      __syncthreads();
-      for (int s = w; s < ni; s += NW) {
-        const double4 pi = a.cell_p[oi + s], mi = a.cell_m[oi + s];
-        const int i = a.cell_i[oi + s], typi = (int)mi.w;
-        const int eo = a.ex_off[i], en = a.ex_num[i];
-        int nf = rowf[s], nr = rowr[s];
-        int *row = a.jforce + (size_t)i * a.cap;
-        for (int b0 = 0; b0 < nt; b0 += 64) {
-          const int e = b0 + lane;
-          bool keep = false, inter = false;
-          int j = 0, t = 0;
-          if (e < nt) {
-            j = ti[e];
-            if (j != i) {
-              const double4 pj = tp[e], mj = tm[e];
-              double dx, dy, dz;
-              const double r2 =
-                  min_image_sep(a.cell, a.pimd, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z, mi.x, mi.y, mi.z, mj.x, mj.y, mj.z,
-                                dx, dy, dz);
-              t = pair_index(a.pt.ntype, typi, (int)mj.w);
-              if (r2 < a.pt.cutskin2[t]) {
-                bool excl = false;
-                for (int k = 0; k < en; k++) excl |= (a.ex_j[eo + k] == j);
-                if (!excl) {
-                  keep = j < i;
-                  inter = (a.full || j < i) && (a.pt.lj[t] || (pi.w * pj.w != 0.0));
-                }
-              }
-            }
-          }
-          const uint64_t mi2 = __ballot(inter);
-          if (inter) {
-            const int p = nf + __popcll(mi2 & below);
-            if (p < a.cap) row[p] = j | (t << ENTRY_SHIFT);
-          }
-          nf += __popcll(mi2);
-          nr += __popcll(__ballot(keep));
-        }
-        if (lane == 0) {
-          rowf[s] = nf;
-          rowr[s] = nr;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  int sum = 0;
-  for (int s = threadIdx.x; s < ni; s += blockDim.x) {
-    const int i = a.cell_i[oi + s], nf = rowf[s];
-    a.nforce[i] = nf;
-    if (nf > a.cap) atomicMax(a.overflow, nf);
-    sum += rowr[s];
-  }
-  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
-  if (lane == 0) red[w] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int k = 0; k < NW; k++) t += red[k];
-    atomicAdd(a.overflow + 1, t);
-  }
-}
-
-// nw wavefronts per cell's workgroup (4, 8 or 16): more of them keep more
-// loads in flight; each site's row is still written by one wavefront, in
-// stencil order.
-template <int NW>
-void launch_list_cells_w(const ListArgs &a, int halfwidth, int ncell, hipStream_t st) {
-  if (halfwidth == 2)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_list_cells<2, NW>), dim3(ncell), dim3(64 * NW), 0, st, a);
-  else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_list_cells<1, NW>), dim3(ncell), dim3(64 * NW), 0, st, a);
-}
-
-hipError_t launch_list_cells(const ListArgs &a, int halfwidth, int ncell, int nw, hipStream_t st) {
-  if (nw >= 16) launch_list_cells_w<16>(a, halfwidth, ncell, st);
-  else if (nw >= 8) launch_list_cells_w<8>(a, halfwidth, ncell, st);
-  else launch_list_cells_w<4>(a, halfwidth, ncell, st);
-  return hipGetLastError();
-}
-
-// Sorts each list row ascending by site index (one workgroup per row,
-// bitonic sort in LDS over n2 >= cap keys): the link-cell build then yields
-// the same rows, in the same order, as the ascending scan.
-__global__ void __launch_bounds__(256) k_sort_rows(int cap, int n2, const int *nfull, const int *nforce, int *jfull,
-                                                   int *jforce) {
-  extern __shared__ int keys[];
-  const int i = blockIdx.x, tid = threadIdx.x;
-  for (int which = 0; which < 2; which++) {
-    int *row = (which == 0 ? jfull : jforce) + (size_t)i * cap;
-    const int cnt = which == 0 ? nfull[i] : nforce[i];
-    int m = 64;  // this row's sort width: a power of two >= cnt, <= n2
-    while (m < cnt && m < n2) m <<= 1;
-    for (int k = tid; k < m; k += blockDim.x) keys[k] = k < cnt ? row[k] : ENTRY_MASK | 0x7f000000;
-    __syncthreads();
-    for (int len = 2; len <= m; len <<= 1) {
-      for (int half = len >> 1; half > 0; half >>= 1) {
-        for (int k = tid; k < m; k += blockDim.x) {
-          const int p = k ^ half;
-          if (p > k) {
-            const int a = keys[k], b = keys[p];
-            const bool up = (k & len) == 0;
-            const bool swap = up ? ((a & ENTRY_MASK) > (b & ENTRY_MASK)) : ((a & ENTRY_MASK) < (b & ENTRY_MASK));
-            if (swap) {
-              keys[k] = b;
-              keys[p] = a;
-            }
-          }
-        }
-        __syncthreads();
-      }
-    }
-    for (int k = tid; k < cnt; k += blockDim.x) row[k] = keys[k];
-    __syncthreads();
-  }
+// The records in site order, for the build without cells.
+__global__ void __launch_bounds__(256) k_list_records(ListArgs a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < a.N) list_record(a, i, i);
 }
 
 // Orders the LDS writes of a wavefront before its other lanes read them
@@ -778,6 +576,187 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The force list (make_lnk_lst.c:37-355, lnk_ver_gen_pad in
+// verlist_control.c:1738-2254): one wavefront per site, in candidate order.
+// H > 0: link cells of fractional space at least r_list / H wide, at least
+// 2H + 1 per axis, so that the (2H + 1)^3 cells around a site's cell hold
+// every site within the list radius, each once; a row of 2H + 1 cells along a
+// is one run of the cell order, or two where it wraps.  H = 0: every site.
+//
+// Each candidate is first tested in FP32 on its cell fractions (cubic and
+// orthorhombic cells: the nearest image of bead 1 is never farther than the
+// image that the list's test takes, so a candidate past the largest
+// cut+skin, with room for the rounding, cannot be on the list).  The few
+// that pass, about a quarter, queue in LDS and 64 at a time take the
+// reference's own test (min_image_sep, its image and cut+skin, the same
+// bits), then the exclusion list; ballots append the interacting pairs to
+// the row (every j != i, or j < i for the half list) in candidate order.  The
+// reference's half-list pairs (j < i, every type pair) are counted into nfull.
+//
+// A workgroup per cell with the FP64 test for every candidate, staged in LDS
+// a stencil row at a time, had 125 workgroups for 1024 q-TIP4P/F at P = 8 and
+// 320 us of kernel for 4096 of them at 31 % VALU busy.  The list stage of a
+// rebuilding call, before -> now: 671 -> 105 us and 429 -> 216 us.
+constexpr int LIST_WAVES = 4;
+template <int H>
+__global__ void __launch_bounds__(64 * LIST_WAVES) k_list_rows(ListArgs a) {
+#pragma clang fp contract(off)
+  __shared__ int queue[LIST_WAVES][128];
+  constexpr int W = 2 * H + 1;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int s = blockIdx.x * LIST_WAVES + w;
+  if (s >= a.N) return;  // uniform over the wavefront; no barriers below
+  const double4 pi = a.cell_p[s], mi = a.cell_m[s];
+  const float4 fi = a.cell_f[s];
+  const int i = a.cell_i[s], typi = (int)mi.w;
+  const int eo = a.ex_off[i], en = a.ex_num[i];
+  const float h0 = (float)a.cell.h[0], h1 = (float)a.cell.h[4], h2 = (float)a.cell.h[8], lim = a.lim2;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int *row = a.jrow + (size_t)i * a.cap;
+  int nf = 0, nr = 0, qn = 0;
+  auto flush = [&](int n) {
+    bool keep = false, inter = false;
+    int j = 0, t = 0;
+    if (lane < n) {
+      const int e = queue[w][lane];
+      const double4 pj = a.cell_p[e], mj = a.cell_m[e];
+      j = a.cell_i[e];
+      double dx, dy, dz;
+      const double r2 = min_image_sep(a.cell, a.pimd, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z, mi.x, mi.y, mi.z, mj.x, mj.y,
+                                      mj.z, dx, dy, dz);
+      t = pair_index(a.pt.ntype, typi, (int)mj.w);
+      if (r2 < a.pt.cutskin2[t]) {
+        bool excl = false;
+        for (int k = 0; k < en; k++) excl |= (a.ex_j[eo + k] == j);
+        if (!excl) {
+          keep = j < i;
+          inter = (a.full || j < i) && (a.pt.lj[t] || (pi.w * pj.w != 0.0));
+        }
+      }
+    }
+    const uint64_t mk = __ballot(inter);
+    if (inter) {
+      const int p = nf + __popcll(mk & below);
+      if (p < a.cap) row[p] = j | (t << ENTRY_SHIFT);
+    }
+    nf += __popcll(mk);
+    nr += __popcll(__ballot(keep));
+  };
+  auto feed = [&](int start, int len) {  // uniform over the wavefront
+    float4 fn = a.cell_f[start + min(lane, len - 1)];
+    for (int k = 0; k < len; k += 64) {
+      const float4 f = fn;
+      fn = a.cell_f[start + min(k + 64 + lane, len - 1)];
+      const int e = start + k + lane;
+      float d0 = f.x - fi.x, d1 = f.y - fi.y, d2 = f.z - fi.z;
+      d0 = (d0 - rintf(d0)) * h0;
+      d1 = (d1 - rintf(d1)) * h1;
+      d2 = (d2 - rintf(d2)) * h2;
+      const bool in = k + lane < len && e != s && d0 * d0 + d1 * d1 + d2 * d2 < lim;
+      const uint64_t mk = __ballot(in);
+      if (in) queue[w][qn + __popcll(mk & below)] = e;
+      qn += __popcll(mk);
+      wave_sync();
+      if (qn >= 64) {
+        flush(64);
+        const int rest = queue[w][64 + lane];
+        wave_sync();
+        queue[w][lane] = rest;
+        wave_sync();
+        qn -= 64;
+      }
+    }
+  };
+  if constexpr (H == 0) {
+    feed(0, a.N);
+  } else {
+    // lane r holds the runs of stencil row r
+    int s0 = 0, n0 = 0, s1 = 0, n1 = 0;
+    {
+      const int c = a.site_cell[i], ca = c % a.nc[0], cb = (c / a.nc[0]) % a.nc[1], cc = c / (a.nc[0] * a.nc[1]);
+      if (lane < W * W) {
+        const int nb = (cb + lane % W - H + a.nc[1]) % a.nc[1], nz = (cc + lane / W - H + a.nc[2]) % a.nc[2];
+        const int base = (nz * a.nc[1] + nb) * a.nc[0], lo = ca - H, hi = ca + H;
+        auto run = [&](int f, int l, int &st, int &n) {  // cells f .. l of the row
+          st = a.cell_start[base + f];
+          n = a.cell_start[base + l] + a.cell_cnt[base + l] - st;
+        };
+        if (lo < 0) {
+          run(lo + a.nc[0], a.nc[0] - 1, s0, n0);
+          run(0, hi, s1, n1);
+        } else if (hi >= a.nc[0]) {
+          run(lo, a.nc[0] - 1, s0, n0);
+          run(0, hi - a.nc[0], s1, n1);
+        } else {
+          run(lo, hi, s0, n0);
+        }
+      }
+    }
+    for (int r = 0; r < W * W; r++) {
+      const int b0 = __builtin_amdgcn_readlane(s0, r), l0 = __builtin_amdgcn_readlane(n0, r);
+      const int b1 = __builtin_amdgcn_readlane(s1, r), l1 = __builtin_amdgcn_readlane(n1, r);
+      if (l0 > 0) feed(b0, l0);
+      if (l1 > 0) feed(b1, l1);
+    }
+  }
+  if (qn > 0) flush(qn);
+  if (lane == 0) {
+    a.nforce[i] = nf;
+    a.nfull[i] = nr;
+  }
+}
+
+hipError_t launch_list_rows(const ListArgs &a, int halfwidth, hipStream_t st) {
+  const dim3 grid((a.N + LIST_WAVES - 1) / LIST_WAVES), block(64 * LIST_WAVES);
+  if (halfwidth == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_list_rows<2>), grid, block, 0, st, a);
+  else if (halfwidth == 1) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_list_rows<1>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_list_rows<0>), grid, block, 0, st, a);
+  return hipGetLastError();
+}
+
+// The longest row if one outgrew its width, and the pair count (one
+// workgroup; an atomic per row on one address costs more than the rows).
+__global__ void __launch_bounds__(1024) k_list_counts(ListArgs a) {
+  __shared__ int mx[16], sm[16];
+  int m = 0, n = 0;
+  for (int i = threadIdx.x; i < a.N; i += 1024) {
+    const int f = a.nfull[i], r = a.ref_only ? f : a.nforce[i];
+    m = max(m, r);
+    n += f;
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    m = max(m, __shfl_xor(m, off, 64));
+    n += __shfl_xor(n, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    mx[threadIdx.x >> 6] = m;
+    sm[threadIdx.x >> 6] = n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) {
+      m = max(m, mx[w]);
+      n += sm[w];
+    }
+    a.overflow[0] = m > a.cap ? m : 0;
+    a.overflow[1] = n;
+  }
+}
+
+// The state a list is built from, kept for the checks and the reference list.
+__global__ void __launch_bounds__(256) k_list_keep(int N, const double *b0, const double *b1, const double *b2,
+                                                   const double *m0, const double *m1, const double *m2, double *x0,
+                                                   double *y0, double *z0, double *xm0, double *ym0, double *zm0) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  x0[i] = b0[i];
+  y0[i] = b1[i];
+  z0[i] = b2[i];
+  xm0[i] = m0[i];
+  ym0[i] = m1[i];
+  zm0[i] = m2[i];
+}
+
 // Splits every force-list row, stably, into the entries whose pair lies
 // inside its cutoff at the build positions (the centroid reference xmod with
 // beads, bead 1 without), then the rest of the list shell, into out.  The
@@ -785,16 +764,16 @@ __device__ __forceinline__ void wave_sync() {
 // time; grouped like this, the pairs of one iteration mostly agree on the
 // cutoff test and the lanes of a wavefront seldom idle.  One wavefront per
 // row.
-__global__ void __launch_bounds__(256) k_split_rows(ListArgs a, int *out) {
+__global__ void __launch_bounds__(256) k_split_rows(ListArgs a) {
   // the inside flags of a row's chunks, kept from the counting pass for the
   // placing pass (rows of up to SPLIT_CHUNKS chunks; longer rows test again)
   __shared__ uint64_t msk[4][SPLIT_CHUNKS];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i = (int)(((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   if (i >= a.N) return;  // uniform over the wavefront
-  const int cnt = a.nforce[i];
-  const int *row = a.jforce + (size_t)i * a.cap;
-  int *dst = out + (size_t)i * a.cap;
+  const int cnt = min(a.nforce[i], a.cap);  // a row that outgrew its width: the build is done again
+  const int *row = a.jrow + (size_t)i * a.cap;
+  int *dst = a.jforce + (size_t)i * a.cap;
   const double xi = a.pimd ? a.xm[i] : a.bx[i], yi = a.pimd ? a.ym[i] : a.by[i], zi = a.pimd ? a.zm[i] : a.bz[i];
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   auto inside = [&](int e) {

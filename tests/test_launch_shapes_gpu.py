@@ -99,3 +99,30 @@ def test_chain_lengths(len_nhc):
     assert np.abs(chains - st).max() < 1e-9 * np.abs(st).max()
     assert abs(ec[3] - eco[3]) < 1e-9 * np.abs(eco).max()
     eng.close()
+
+
+# the force list by cells and by the scan over every site, orthorhombic (FP32
+# test first) and triclinic (none), rows that fill a queue and that do not
+@pytest.mark.parametrize("mode", ["brute", "cells"])
+@pytest.mark.parametrize("nmol, P, cell", [(2, 1, None), (65, 4, None), (300, 1, None), (700, 2, None),
+                                           (300, 2, ((1.0, 0.15, 0.0), (0.0, 1.0, 0.1), (0.05, 0.0, 1.0)))])
+def test_list_rows(monkeypatch, mode, nmol, P, cell):
+    from piny_amd.engine import Engine
+    monkeypatch.setenv("PMX_LIST", mode)
+    rc = 3.0 if nmol > 2 else 2.0
+    c = w.small_config(w.SPC_FW, nmol=nmol, P=P, seed=nmol, cutoff=rc)
+    if cell is not None:
+        c = w.with_cell(c, np.array(cell) * c.system.box)
+    x, y, z = c.x + 40.0, c.y - 55.0, c.z * 1.0  # outside the cell
+    flags = abi.PMX_EVAL_PIMD if P > 1 else 0
+    eng = Engine(c.system, x, y, z)
+    eng.set_positions(x, y, z)
+    e = eng.energy_control(flags)
+    o = Oracle(c.system, x, y, z)
+    eo, fo, _ = o.energy_control(x, y, z, flags)
+    assert e["nver"] == eo["nver"]
+    f = eng.forces()
+    assert np.sqrt(((f - fo) ** 2).sum() / (fo ** 2).sum()) < FP64_TOL
+    for a, b in zip(eng.verlet_list(), o.verlet_list()):
+        assert np.array_equal(a, b)
+    eng.close()
