@@ -119,9 +119,10 @@ struct pmx_ctx {
   double2 *ew_sk = nullptr;
   // binned PME: tiling, per-item data, bins, halo boxes
   PmeArgs pa{};
-  int *item_s = nullptr, *item_tile = nullptr, *item_pos = nullptr, *bin_cnt = nullptr, *bin_off = nullptr,
-      *sorted = nullptr;
-  double *item_f = nullptr, *hbuf = nullptr;
+  int *bin_cnt = nullptr, *bin_off = nullptr;
+  int2 *item_kp = nullptr, *item_s = nullptr;
+  double4 *item_f = nullptr;
+  double *hbuf = nullptr;
   // per-block partial sums of every stage, then accumulators [P][ACC_NUM] + ake
   double *part = nullptr;
   size_t part_n = 0;       // doubles of part
@@ -158,7 +159,7 @@ struct pmx_ctx {
   // launch shapes (set at creation, changed by pmx_autotune): PME tile
   // caps, wavefronts of the pair kernels, list build (0 by size, 1 plain
   // scan, 2 link cells)
-  int tile_cap[3] = {16, 16, 8};
+  int tile_cap[3] = {0, 0, 0};  // upper bounds of the PME tile; 0: auto_tile_caps
   int pair_waves = 4096;
   int list_mode = 0;
   hipEvent_t ready = nullptr;  // list stage done (batched calls)
@@ -332,6 +333,49 @@ constexpr int MAX_LIST_CELLS = 1 << 18;
     if (rc_) return rc_; \
   } while (0)
 
+// Items of a tile are sorted by plane (bins of one tile and plane) while a
+// bead's bins stay within bounds.  Whole tiles as bins would do for the
+// atomics' spread, but the counting sort's atomics then meet on few addresses
+// (15009 charges, P = 1: 24 instead of 4.5 us).
+bool pme_plane_bins(const int T[3], const int K[3]) {
+  return T[2] >= 2 && T[2] <= PME_ZB_MAX && (long)(K[0] / T[0]) * (K[1] / T[1]) * K[2] <= PME_NBIN_MAX;
+}
+
+// The matrix-core spread needs plane bins, tiles whose patch, T + n - 1 points
+// wide along a and b, fits a 16 x 16 accumulator, and an order it is built
+// for.  It pays from some 10^5 charges on: a wavefront per tile is one long
+// chain, and a box that does not fill the chip with them waits for it (both
+// spreads on the same tiles, matrix cores and LDS atomics: 54 and 64 us at
+// 393216 charges, 71 and 95 us at 576048, 19 and 13 us at 24576, 20 and 10 us
+// at 15009).
+bool pme_mm(int n, long items, const int T[3], const int K[3]) {
+  return n <= 8 && items >= PME_MM_ITEMS && T[0] + n - 1 <= 16 && T[1] + n - 1 <= 16 && pme_plane_bins(T, K);
+}
+
+// Tile caps when none are given: along a and b the widest tile of the
+// matrix-core spread that is at least n - 1 wide (the fold then sums two boxes
+// an axis), along c up to 12 planes (at 24 the matrix-core spread of 393216
+// charges has too few wavefronts, 68 us; at 8 and 12 it takes 55 and 54 us),
+// 8 for the boxes of the other spread, which smaller tiles deal over more of
+// the chip: the gather of 15009 charges, P = 1, took 27 us on 16 x 16 x 8
+// tiles, 13 us on 8 x 8 x 12, 9 us on 8 x 8 x 8.  Grids with no such tile
+// keep 16 x 16 x 8.
+void auto_tile_caps(const Setup &s, int n, int cap[3]) {
+  auto divisor = [](int K, int lo, int hi) {  // the largest divisor of K in [lo, hi], or 0
+    for (int t = std::min(hi, K); t >= lo; t--)
+      if (K % t == 0) return t;
+    return 0;
+  };
+  const int lo = n - 1, t0 = divisor(s.ngrid[0], lo, 17 - n), t1 = divisor(s.ngrid[1], lo, 17 - n);
+  int t2 = divisor(s.ngrid[2], lo, (long)s.P * (long)s.ichrg.size() >= PME_MM_ITEMS ? 12 : std::max(lo, 8));
+  cap[0] = cap[1] = 16;
+  cap[2] = 8;
+  if (n > 8 || !t0 || !t1 || !t2) return;
+  cap[0] = t0;
+  cap[1] = t1;
+  cap[2] = t2;
+}
+
 // Chooses the PME tile (the largest divisors of the grid below the caps
 // whose halo box fits the LDS of one workgroup), allocates the binning
 // buffers and
@@ -357,12 +401,13 @@ int setup_pme_tiles(pmx_ctx *c) {
   a.f32 = c->pme_f32;
   // tiles divide the grid, so every tile is whole and a support of n points
   // starting in a tile reaches at most ceil((n-1)/T) tiles beyond it
-  int cap[3] = {c->tile_cap[0], c->tile_cap[1], c->tile_cap[2]};
   auto divisor_below = [](int K, int m) {
     int t = std::max(1, std::min(m, K));
     while (K % t) t--;
     return t;
   };
+  int cap[3] = {c->tile_cap[0], c->tile_cap[1], c->tile_cap[2]};
+  if (cap[0] == 0) auto_tile_caps(s, n, cap);
   int T[3];
   for (;;) {
     for (int d = 0; d < 3; d++) T[d] = divisor_below(s.ngrid[d], cap[d]);
@@ -380,7 +425,7 @@ int setup_pme_tiles(pmx_ctx *c) {
     a.mT1 = magic(a.T[1]);
     bool ok = true;
     for (int d = 0; d < 3; d++) a.nbr[d] = 1 + (n - 1 + a.T[d] - 1) / a.T[d];
-    ok = ok && (size_t)a.nt[0] * a.nt[1] * a.nt[2] * sizeof(int) <= 65536;  // LDS histogram of k_pme_bin
+    ok = ok && (size_t)a.nt[0] * a.nt[1] * a.nt[2] * (pme_plane_bins(T, s.ngrid) ? T[2] : 1) <= (size_t)PME_NBIN_MAX;
     ok = ok && pme_lds_bytes(a, true) <= FFT_LDS_MAX && pme_lds_bytes(a, false) <= FFT_LDS_MAX;
     // 32-bit element offsets into one bead's halo boxes
     ok = ok && (size_t)a.nt[0] * a.nt[1] * a.nt[2] * a.hvol < (1ull << 31);
@@ -398,27 +443,27 @@ int setup_pme_tiles(pmx_ctx *c) {
   a.ntile = a.nt[0] * a.nt[1] * a.nt[2];
   a.gstride = c->gstride;
   const size_t nitem = (size_t)s.P * a.nchrg;
+  a.zb = pme_plane_bins(T, s.ngrid) ? T[2] : 1;
+  a.mm = pme_mm(n, (long)s.P * a.nchrg, T, s.ngrid);
+  a.nbin = a.ntile * a.zb;
   if (!c->item_s) {
-    TRY_RC(dalloc(c, &c->item_s, 3 * nitem));
-    TRY_RC(dalloc(c, &c->item_f, 3 * nitem));
-    TRY_RC(dalloc(c, &c->item_tile, nitem));
-    TRY_RC(dalloc(c, &c->item_pos, nitem));
-    TRY_RC(dalloc(c, &c->sorted, nitem));
+    TRY_RC(dalloc(c, &c->item_s, nitem));
+    TRY_RC(dalloc(c, &c->item_f, nitem));
+    TRY_RC(dalloc(c, &c->item_kp, nitem));
   }
-  dfree(c, c->bin_cnt);  // a second tiling (autotuner) replaces the tile-sized buffers
-  dfree(c, c->bin_off);
+  dfree(c, c->bin_cnt);
+  dfree(c, c->bin_off);  // a second tiling (autotuner) replaces the tile-sized buffers
   dfree(c, c->hbuf);
-  TRY_RC(dalloc(c, &c->bin_cnt, (size_t)s.P * a.ntile));
-  TRY_RC(dalloc(c, &c->bin_off, (size_t)s.P * a.ntile));
+  TRY_RC(dalloc(c, &c->bin_cnt, (size_t)s.P * a.nbin));
+  HIPCHK(hipMemsetAsync(c->bin_cnt, 0, (size_t)s.P * a.nbin * sizeof(int), c->st));  // setup, never captured
+  TRY_RC(dalloc(c, &c->bin_off, (size_t)s.P * (a.nbin + 1)));
   TRY_RC(dalloc(c, &c->hbuf, (size_t)s.P * a.ntile * a.hvol));
   a.hbuf = c->hbuf;
-  a.item_s = c->item_s;
-  a.item_f = c->item_f;
-  a.item_tile = c->item_tile;
-  a.item_pos = c->item_pos;
-  a.sorted = c->sorted;
-  a.bin_cnt = c->bin_cnt;
-  a.bin_off = c->bin_off;
+  a.cnt = c->bin_cnt;
+  a.kp = c->item_kp;
+  a.rfs = c->item_f;
+  a.ris = c->item_s;
+  a.off = c->bin_off;
   a.grid = c->grid;
   a.q = c->q;
   a.ichrg = c->ichrg;
@@ -1544,15 +1589,7 @@ int launch_pme(pmx_ctx *c, hipStream_t sk) {
   a.rx = c->frec;
   a.ry = c->frec + NP;
   a.rz = c->frec + 2 * NP;
-  const size_t nitem = (size_t)P * nchrg, nbin = (size_t)P * a.ntile;
-  hipLaunchKernelGGL(k_fill_int, dim3(blocks(nbin)), dim3(256), 0, sk, c->bin_cnt, 0, nbin);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_pme_bin, dim3(blocks(nchrg), P), dim3(256), (size_t)a.ntile * sizeof(int), sk, a);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_pme_scan, dim3(P), dim3(256), 0, sk, a);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_pme_scatter, dim3(blocks(nitem)), dim3(256), 0, sk, a);
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_pme_bin(a, sk));
   HIPCHK(launch_pme_spread(a, sk));
   FftArgs f{};
   f.P = P;
@@ -2648,7 +2685,7 @@ int pmx_autotune(pmx_ctx *c, unsigned flags, int reps, int *choice) {
   }
   // PME tiles (stage 2, k space)
   if (c->pme) {
-    const int cand[][3] = {{16, 16, 8}, {8, 8, 8}, {16, 8, 8}, {16, 16, 4}, {32, 16, 8}, {32, 8, 8}, {8, 8, 4}};
+    const int cand[][3] = {{0, 0, 0}, {16, 16, 8}, {8, 8, 8}, {8, 8, 16}, {8, 8, 32}, {10, 10, 16}, {16, 8, 8}};
     int best[3] = {c->tile_cap[0], c->tile_cap[1], c->tile_cap[2]};
     double tbest = 1e300;
     for (const auto &cap : cand) {
@@ -2758,7 +2795,7 @@ int pmx_batch_autotune(pmx_batch *b, unsigned flags, int reps, int *choice) {
     if (choice) choice[0] = best;
   }
   {
-    const int cand[][3] = {{16, 16, 8}, {8, 8, 8}, {16, 8, 8}, {8, 8, 4}, {32, 16, 8}, {16, 16, 16}};
+    const int cand[][3] = {{0, 0, 0}, {16, 16, 8}, {8, 8, 8}, {8, 8, 16}, {8, 8, 32}, {10, 10, 16}};
     int best = 0;
     double tbest = 1e300;
     for (int k = 0; k < (int)(sizeof cand / sizeof cand[0]); k++) {

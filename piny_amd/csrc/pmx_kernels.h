@@ -130,11 +130,17 @@ struct PmeArgs {
   const double *q;
   const int *ichrg;
   Cell cell;
-  int *item_s;         // [P*nchrg][3] first support point per axis (0-based)
-  double *item_f;      // [P*nchrg][3] fractional grid offset per axis
-  int *item_tile, *item_pos;
-  int *bin_cnt, *bin_off;  // [P*ntile]
-  int *sorted;         // [P*nchrg] item ids in bin order
+  // bins: zb per tile (T[2]: the tile's items are sorted by the plane of their
+  // first support point; or 1), nbin per bead; mm: k_pme_spread_mm spreads
+  int zb, nbin, mm;
+  int *cnt;            // [P*nbin] items per bin; zero between calls
+  int2 *kp;            // [nchrg*P] bin of an item and its place there
+  // items sorted by bin, bead-major [P][nchrg]: fractional grid offsets and
+  // charge (4 values of the grid type), and (first support point per axis, 10
+  // bits each; charge index)
+  void *rfs;
+  int2 *ris;
+  int *off;            // [P][nbin + 1] first sorted item of a bin
   void *hbuf;          // [P*ntile*hvol] halo boxes of spread charge (grid type)
   void *grid;          // [P*gstride] (grid type)
   double *rx, *ry, *rz;  // gather: the k-space force of every (charge, bead), bead-major [P][N]
@@ -155,6 +161,10 @@ struct EwaldArgs {
   double *part;       // partial rows, FFT_NV values
 };
 constexpr int EWALD_BLOCK = 256;
+
+constexpr int PME_NBIN_MAX = 1 << 17;  // bins of one bead
+constexpr long PME_MM_ITEMS = 100000;  // (charge, bead) items from which the matrix-core spread pays
+constexpr int PME_ZB_MAX = 63;       // planes of a tile whose item offsets one wavefront's lanes hold
 
 constexpr int FFT_MAX_PASSES = 12;
 constexpr int FFT_MAX_PLANE = 4096;       // complex values per plane of the smaller class
@@ -386,9 +396,6 @@ __global__ void k_list_counts(ListArgs a);
 __global__ void k_list_keep(int N, const double *b0, const double *b1, const double *b2, const double *m0,
                             const double *m1, const double *m2, double *x0, double *y0, double *z0, double *xm0,
                             double *ym0, double *zm0);
-__global__ void k_pme_bin(PmeArgs a);
-__global__ void k_pme_scan(PmeArgs a);
-__global__ void k_pme_scatter(PmeArgs a);
 __global__ void k_fill_int(int *p, int v, size_t n);
 __global__ void k_fill_double(double *p, double v, size_t n);
 __global__ void k_reduce_partials(RedArgs a);
@@ -476,6 +483,7 @@ int pair_tab_grid_x(int N, int max_waves);
 constexpr int PAIR_MAX_WAVES = 16384;  // the largest pair grid the autotuner tries
 // LDS bytes of the spread and gather workgroups for a given tiling
 size_t pme_lds_bytes(const PmeArgs &a, bool gather);
+hipError_t launch_pme_bin(const PmeArgs &a, hipStream_t st);
 hipError_t launch_pme_spread(const PmeArgs &a, hipStream_t st);
 hipError_t launch_pme_gather(const PmeArgs &a, hipStream_t st);
 hipError_t launch_pme_phi(const PmeArgs &a, hipStream_t st);

@@ -6,10 +6,13 @@
 // over the half-space sphere list (:367-430) and the force gather (:500-560).
 // The MI355X layout differs from the reference's loop order:
 //  - every (charge, bead) is binned by the grid tile holding the first point
-//    of its support (k_pme_bin / k_pme_scan / k_pme_scatter, a counting sort);
-//  - one workgroup per (tile, bead) spreads the charges of its bin, one lane
-//    per charge, into an LDS halo box of (T + n - 1)^3 points with LDS
-//    atomics and writes the box out once (no global atomics, no grid clear);
+//    of its support, and within the tile by that point's plane (a counting
+//    sort: k_pme_count, k_pme_scan, k_pme_place, or k_pme_sort alone);
+//  - the spread is a contraction: per plane of a tile, outer products of the
+//    charges' weights along a and b, summed on the FP64 matrix cores into a
+//    16 x 16 patch held in registers (k_pme_spread_mm), written out once (no
+//    atomics, no grid clear).  Orders above 8, and grids without a fitting
+//    tile, take LDS atomics into a halo box instead (k_pme_spread);
 //  - the forward FFT sums, as it loads each grid plane, every point's own
 //    box and the overhang of the boxes below it (the fold into the periodic
 //    grid never goes through memory);
@@ -83,109 +86,328 @@ __device__ __forceinline__ void tile_origin(const PmeArgs &a, int tl, int &o0, i
 
 // --- binning -----------------------------------------------------------------
 
-// one thread per item it = bead*nchrg + charge (grid: charge chunks x beads):
-// fractional grid coordinates (ewald3d_pme.c:241-262, 270-276), first support
-// point per axis, and the item's slot in its bin.  Slots are counted in an
-// LDS histogram per workgroup first, so each (block, tile) pair makes one
-// global atomic instead of one per item.
-__global__ void __launch_bounds__(256) k_pme_bin(PmeArgs a) {
-  extern __shared__ int hist[];  // [ntile]
-  const int b = blockIdx.y, ic = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool act = ic < a.nchrg;
-  for (int t = threadIdx.x; t < a.ntile; t += blockDim.x) hist[t] = 0;
-  __syncthreads();
-  const int it = b * a.nchrg + ic;
-  int tile = 0, lpos = 0;
-  if (act) {
-    const size_t ib = (size_t)a.ichrg[ic] * a.P + b;
-    const double x = a.x[ib], y = a.y[ib], z = a.z[ib];
-    const double *hi = a.cell.hi;
-    double s[3];
-    s[0] = x * hi[0] + y * hi[3] + z * hi[6];
-    s[1] = x * hi[1] + y * hi[4] + z * hi[7];
-    s[2] = x * hi[2] + y * hi[5] + z * hi[8];
-    int tcoord[3];
+// a (charge, bead) item: fractional grid offset per axis and the charge
+template <typename T>
+struct Rec;
+template <>
+struct Rec<double> {
+  using V = double4;
+};
+template <>
+struct Rec<float> {
+  using V = float4;
+};
+
+// Item (charge ic, bead b): the fractional grid coordinates
+// (ewald3d_pme.c:241-262, 270-276), formed in FP64; the first support point
+// per axis, 10 bits each, with the charge's index; and the item's bin: its
+// tile and, with zb > 1, its plane within the tile.
+template <typename T>
+__device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typename Rec<T>::V &f, int2 &si) {
+  const size_t ib = (size_t)a.ichrg[ic] * a.P + b;
+  const double x = a.x[ib], y = a.y[ib], z = a.z[ib];
+  const double *hi = a.cell.hi;
+  double s[3], fr[3];
+  s[0] = x * hi[0] + y * hi[3] + z * hi[6];
+  s[1] = x * hi[1] + y * hi[4] + z * hi[7];
+  s[2] = x * hi[2] + y * hi[5] + z * hi[8];
+  int s0[3];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      const int K = a.K[d];
-      const double t = s[d] - nint_d((s[d] - 0.5));
-      const double sc = t * (double)K;
-      int ig = (int)(sc);
-      const double frac = sc - (double)ig;
-      // support points (0-based) ig - n + 1 .. ig, periodic; ig = K (a
-      // coordinate rounding onto the upper face) is the same set as ig = 0
-      ig = ((ig % K) + K) % K;
-      int s0 = ig - a.n + 1;
-      s0 = ((s0 % K) + K) % K;
-      a.item_f[3 * (size_t)it + d] = frac;
-      a.item_s[3 * (size_t)it + d] = s0;
-      tcoord[d] = s0 / a.T[d];
+  for (int d = 0; d < 3; d++) {
+    const int K = a.K[d];
+    const double t = s[d] - nint_d((s[d] - 0.5));
+    const double sc = t * (double)K;
+    int ig = (int)(sc);
+    fr[d] = sc - (double)ig;
+    // support points (0-based) ig - n + 1 .. ig, periodic; ig = K (a
+    // coordinate rounding onto the upper face) is the same set as ig = 0
+    ig = ((ig % K) + K) % K;
+    const int g = ig - a.n + 1;
+    s0[d] = ((g % K) + K) % K;
+  }
+  f.x = (T)fr[0];
+  f.y = (T)fr[1];
+  f.z = (T)fr[2];
+  f.w = (T)a.q[a.ichrg[ic]];
+  si = make_int2(s0[0] | (s0[1] << 10) | (s0[2] << 20), ic);
+  const int tc = s0[2] / a.T[2], tile = (tc * a.nt[1] + s0[1] / a.T[1]) * a.nt[0] + s0[0] / a.T[0];
+  return a.zb > 1 ? tile * a.zb + s0[2] - tc * a.T[2] : tile;
+}
+
+// The counting sort of the items by bin.  k_pme_count: one thread per (charge,
+// bead) in the positions' own order; an atomic on the item's bin (some
+// charges to a bin, so the addresses differ) hands out its place there.
+// k_pme_scan: the bins' first places, one workgroup a bead, which leaves the
+// counts zero for the next call.  k_pme_place: every item formed again and
+// written to its place (its 24 bytes cost more to keep than to form).
+template <typename T>
+__global__ void __launch_bounds__(256) k_pme_count(PmeArgs a) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.nchrg * a.P) return;
+  const int c = t / a.P, b = t - c * a.P;
+  typename Rec<T>::V f;
+  int2 si;
+  const int key = pme_item<T>(a, c, b, f, si);
+  a.kp[t] = make_int2(key, atomicAdd(a.cnt + (size_t)b * a.nbin + key, 1));
+}
+
+// exclusive scan over the workgroup's threads of each one's value
+__device__ __forceinline__ int block_scan(int v, int *wsum) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  int inc = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(inc, off, 64);
+    inc += lane >= off ? u : 0;
+  }
+  if (lane == 63) wsum[tid >> 6] = inc;
+  __syncthreads();
+  int run = inc - v;
+  for (int w = 0; w < (tid >> 6); w++) run += wsum[w];
+  return run;
+}
+
+constexpr int SCAN_PER = 4;  // bins a thread takes per round of k_pme_scan
+__global__ void __launch_bounds__(1024) k_pme_scan(PmeArgs a) {
+  __shared__ int wsum[16];
+  __shared__ int total;
+  const int b = blockIdx.x, nbin = a.nbin, tid = threadIdx.x;
+  int *cnt = a.cnt + (size_t)b * nbin, *off = a.off + (size_t)b * (nbin + 1);
+  int base = 0;
+  for (int k0 = 0; k0 < nbin; k0 += 1024 * SCAN_PER) {
+    const int k = k0 + tid * SCAN_PER;
+    int v[SCAN_PER], sum = 0;
+#pragma unroll
+    for (int u = 0; u < SCAN_PER; u++) {
+      v[u] = k + u < nbin ? cnt[k + u] : 0;
+      sum += v[u];
     }
-    tile = (tcoord[2] * a.nt[1] + tcoord[1]) * a.nt[0] + tcoord[0];
-    lpos = atomicAdd(hist + tile, 1);
+    int run = base + block_scan(sum, wsum);
+    if (tid == 1023) total = run + sum;
+#pragma unroll
+    for (int u = 0; u < SCAN_PER; u++)
+      if (k + u < nbin) {
+        off[k + u] = run;
+        cnt[k + u] = 0;
+        run += v[u];
+      }
+    __syncthreads();
+    base = total;
+    __syncthreads();
+  }
+  if (tid == 0) off[nbin] = base;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_pme_place(PmeArgs a) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.nchrg * a.P) return;
+  const int c = t / a.P, b = t - c * a.P;
+  typename Rec<T>::V f;
+  int2 si;
+  (void)pme_item<T>(a, c, b, f, si);
+  const int2 kp = a.kp[t];
+  const size_t o = (size_t)b * a.nchrg + a.off[(size_t)b * (a.nbin + 1) + kp.x] + kp.y;
+  ((typename Rec<T>::V *)a.rfs)[o] = f;
+  a.ris[o] = si;
+}
+
+// The same sort of a small box (up to SORT_ITEMS charges and SORT_BINS bins) in
+// one launch, one workgroup a bead: the items stay in registers, the counts
+// in LDS.
+constexpr int SORT_PER = 2, SORT_ITEMS = 1024 * SORT_PER, SORT_BINS = 8192;
+template <typename T>
+__global__ void __launch_bounds__(1024) k_pme_sort(PmeArgs a) {
+  using V = typename Rec<T>::V;
+  extern __shared__ int hist[];  // [nbin]
+  __shared__ int wsum[16];
+  const int b = blockIdx.x, tid = threadIdx.x, n = a.nchrg, nbin = a.nbin;
+  for (int k = tid; k < nbin; k += 1024) hist[k] = 0;
+  __syncthreads();
+  V f[SORT_PER];
+  int2 si[SORT_PER];
+  int key[SORT_PER], pos[SORT_PER];
+#pragma unroll
+  for (int u = 0; u < SORT_PER; u++) {
+    const int c = tid + u * 1024;
+    if (c < n) {
+      key[u] = pme_item<T>(a, c, b, f[u], si[u]);
+      pos[u] = atomicAdd(hist + key[u], 1);
+    }
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < a.ntile; t += blockDim.x) {
-    const int n = hist[t];
-    hist[t] = n ? atomicAdd(a.bin_cnt + (size_t)b * a.ntile + t, n) : 0;
+  const int per = (nbin + 1023) / 1024, lo = min(nbin, tid * per), hi = min(nbin, lo + per);
+  int sum = 0;
+  for (int k = lo; k < hi; k++) sum += hist[k];
+  int run = block_scan(sum, wsum);
+  int *off = a.off + (size_t)b * (nbin + 1);
+  for (int k = lo; k < hi; k++) {
+    const int v = hist[k];
+    hist[k] = run;
+    off[k] = run;
+    run += v;
   }
+  if (tid == 0) off[nbin] = n;
   __syncthreads();
-  if (act) {
-    a.item_tile[it] = tile;
-    a.item_pos[it] = hist[tile] + lpos;
+#pragma unroll
+  for (int u = 0; u < SORT_PER; u++) {
+    const int c = tid + u * 1024;
+    if (c < n) {
+      const size_t o = (size_t)b * n + hist[key[u]] + pos[u];
+      ((V *)a.rfs)[o] = f[u];
+      a.ris[o] = si[u];
+    }
   }
 }
 
-// exclusive scan of the bin counts of one bead (one workgroup per bead)
-__global__ void __launch_bounds__(256) k_pme_scan(PmeArgs a) {
-  __shared__ int sums[256];
-  const int b = blockIdx.x, tid = threadIdx.x, nt = a.ntile;
-  const int per = (nt + 255) / 256;
-  const int lo = min(nt, tid * per), hi = min(nt, lo + per);
-  const int *cnt = a.bin_cnt + (size_t)b * nt;
-  int s = 0;
-  for (int t = lo; t < hi; t++) s += cnt[t];
-  sums[tid] = s;
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int k = 0; k < 256; k++) {
-      const int v = sums[k];
-      sums[k] = run;
-      run += v;
-    }
+template <typename T>
+hipError_t launch_bin_t(const PmeArgs &a, hipStream_t st) {
+  // one launch while a workgroup holds a bead's items; with more a single
+  // workgroup's time shows (15009 charges, P = 1: 44 us, against 14 in three)
+  if (a.nchrg <= SORT_ITEMS && a.nbin <= SORT_BINS) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_sort<T>), dim3(a.P), dim3(1024), (size_t)a.nbin * sizeof(int), st, a);
+    return hipGetLastError();
   }
-  __syncthreads();
-  int run = b * a.nchrg + sums[tid];
-  for (int t = lo; t < hi; t++) {
-    a.bin_off[(size_t)b * nt + t] = run;
-    run += cnt[t];
-  }
+  const dim3 grid((unsigned)(((size_t)a.nchrg * a.P + 255) / 256)), block(256);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_count<T>), grid, block, 0, st, a);
+  hipLaunchKernelGGL(k_pme_scan, dim3(a.P), dim3(1024), 0, st, a);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_place<T>), grid, block, 0, st, a);
+  return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(256) k_pme_scatter(PmeArgs a) {
-  const int it = blockIdx.x * blockDim.x + threadIdx.x;
-  if (it >= a.P * a.nchrg) return;
-  const int b = it / a.nchrg;
-  a.sorted[a.bin_off[(size_t)b * a.ntile + a.item_tile[it]] + a.item_pos[it]] = it;
+hipError_t launch_pme_bin(const PmeArgs &a, hipStream_t st) {
+  return a.f32 ? launch_bin_t<float>(a, st) : launch_bin_t<double>(a, st);
 }
 
 // --- spread --------------------------------------------------------------------
 
+// the items of bead b's tile tl: [lo, hi) of the bead's sorted items
+__device__ __forceinline__ void tile_items(const PmeArgs &a, int tl, int b, int &lo, int &hi) {
+  const int *off = a.off + (size_t)b * (a.nbin + 1) + (size_t)tl * a.zb;
+  lo = off[0];
+  hi = off[a.zb];
+}
+
 // Weights of one item along the three axes: w[d][m] is the weight of support
 // point s_d + m (M_n index j = n - m); l[d] is s_d relative to the tile origin.
 template <int NI, bool DERIV, typename T>
-__device__ __forceinline__ void item_weights(const PmeArgs &a, int it, const int (&org)[3], T (&w)[3][NI],
+__device__ __forceinline__ void item_weights(const typename Rec<T>::V &f, int s, const int (&org)[3], T (&w)[3][NI],
                                              T (&dw)[3][NI], int (&l)[3]) {
+  const T fr[3] = {f.x, f.y, f.z};
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     T mn[NI + 1], dmn[NI + 1];
-    bspline<NI, DERIV, T>((T)a.item_f[3 * (size_t)it + d], mn, dmn);
-    l[d] = a.item_s[3 * (size_t)it + d] - org[d];
+    bspline<NI, DERIV, T>(fr[d], mn, dmn);
+    l[d] = ((s >> (10 * d)) & 1023) - org[d];
 #pragma unroll
     for (int m = 0; m < NI; m++) {
       w[d][m] = mn[NI - m];
       if (DERIV) dw[d][m] = dmn[NI - m];
+    }
+  }
+}
+
+// The spread as a contraction, one wavefront per (tile, bead).  A charge adds
+// q w_c[m] w_b w_a^T to planes s_c + m of its tile's halo box, so plane by
+// plane four charges with the same s_c (the tile's items come sorted by it)
+// are one rank-4 update of the plane's b x a patch:
+// v_mfma_f64_16x16x4 with A[b][k] = q w_c[m] w_b of charge k and B[k][a] = w_a,
+// zero outside the support.  The n planes that open charges reach live in
+// registers, n rolling accumulators of 16 x 16 (T + n - 1 <= 16); each is
+// stored, rounded to the grid type once, when its last charge has passed.
+// Weights are formed for 16 charges at a time (48 lanes, one axis each) and
+// read back from LDS.
+//
+// The LDS atomics of the form below (216 of FP64 per charge at order 6) took
+// 64 us on the same tiles of 4096 q-TIP4P/F at P = 32 (a 48^3 grid) and 77 us
+// on their 16 x 16 x 8 ones; the matrix cores' part here is 20 us and the
+// vector instructions beside it 17: 53 us.
+typedef double mm_acc __attribute__((ext_vector_type(4)));
+template <int NI, typename T>
+__global__ void __launch_bounds__(64) k_pme_spread_mm(PmeArgs a) {
+  constexpr int NB = 16;
+  __shared__ double sw[NB][3][NI];
+  __shared__ int sl[NB][2];
+  int tl, b;
+  xcd_unit_bead(a.ntile, a.P, tl, b);
+  const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
+  int org[3];
+  tile_origin(a, tl, org[0], org[1], org[2]);
+  const int Tz = a.T[2], H0 = a.H[0], H1 = a.H[1], H01 = H0 * H1;
+  const int *off = a.off + (size_t)b * (a.nbin + 1) + (size_t)tl * Tz;
+  const int offl = off[min(lane, Tz)];  // lane z holds the start of plane z's items (Tz < 64)
+  const int lo = __builtin_amdgcn_readlane(offl, 0), hi = __builtin_amdgcn_readlane(offl, Tz);
+  const typename Rec<T>::V *rf = (const typename Rec<T>::V *)a.rfs + (size_t)b * a.nchrg;
+  const int2 *ri = a.ris + (size_t)b * a.nchrg;
+  T *dst = (T *)a.hbuf + ((size_t)b * a.ntile + tl) * a.hvol;
+  mm_acc acc[NI];
+#pragma unroll
+  for (int m = 0; m < NI; m++) acc[m] = mm_acc{0.0, 0.0, 0.0, 0.0};
+  // this lane's entries of a plane, as byte offsets from the plane
+  unsigned po[4];
+  bool in[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    in[i] = row < H0 && kq + 4 * i < H1;
+    po[i] = (unsigned)((kq + 4 * i) * H0 + row) * (unsigned)sizeof(T);
+  }
+  int pb = lo - NB, p = lo;  // batch in LDS: items pb .. pb + NB - 1
+  // the next batch's items, loaded while the current one is summed
+  typename Rec<T>::V fn{};
+  int sn = 0;
+  auto next = [&](int from) {
+    if (hi > lo) {  // uniform
+      const int c = min(from + row, hi - 1);
+      fn = rf[c];
+      sn = ri[c].x;
+    }
+  };
+  next(lo);
+  for (int z0 = 0; z0 < Tz + NI - 1; z0 += NI) {
+#pragma unroll
+    for (int u = 0; u < NI; u++) {
+      const int z = z0 + u;
+      if (z < Tz + NI - 1) {
+        const int e = z < Tz ? __builtin_amdgcn_readlane(offl, z + 1) : p;
+        while (p < e) {
+          if (p >= pb + NB) {
+            pb = p;
+            __builtin_amdgcn_wave_barrier();
+            if (kq < 3) {
+              T mn[NI + 1], dmn[NI + 1];
+              bspline<NI, false, T>(kq == 0 ? fn.x : kq == 1 ? fn.y : fn.z, mn, dmn);
+              const double q = kq == 2 ? (double)fn.w : 1.0;
+#pragma unroll
+              for (int m = 0; m < NI; m++) sw[row][kq][m] = (double)mn[NI - m] * q;
+            } else {
+              sl[row][0] = (sn & 1023) - org[0];
+              sl[row][1] = ((sn >> 10) & 1023) - org[1];
+            }
+            next(pb + NB);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          }
+          const int n = min(4, min(e, pb + NB) - p), c = min(p - pb + kq, NB - 1);
+          const bool on = kq < n;
+          const int ta = row - sl[c][0], tb = row - sl[c][1];
+          const double wa = sw[c][0][min(max(ta, 0), NI - 1)], wb = sw[c][1][min(max(tb, 0), NI - 1)];
+          const double B = on && (unsigned)ta < (unsigned)NI ? wa : 0.0;
+          const bool bon = on && (unsigned)tb < (unsigned)NI;
+#pragma unroll
+          for (int m = 0; m < NI; m++) {
+            const double A = bon ? wb * sw[c][2][m] : 0.0;
+            acc[(u + m) % NI] = __builtin_amdgcn_mfma_f64_16x16x4f64(A, B, acc[(u + m) % NI], 0, 0, 0);
+          }
+          p += n;
+        }
+        // plane z is complete: lane (row, kq) holds b rows kq + 4 i of column a = row
+        char *plane = (char *)(dst + z * H01);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (in[i]) *(T *)(plane + po[i]) = (T)acc[u][i];
+        acc[u] = mm_acc{0.0, 0.0, 0.0, 0.0};
+      }
     }
   }
 }
@@ -205,7 +427,10 @@ __global__ void __launch_bounds__(spread_lanes<T>() * PME_BLOCK) k_pme_spread(Pm
   const int tid = threadIdx.x;
   for (int k = tid; k < hvol; k += blockDim.x) box[k] = 0.0;
   const size_t bin = (size_t)b * a.ntile + tl;
-  const int lo = a.bin_off[bin], cnt = a.bin_cnt[bin];
+  int lo, hi;
+  tile_items(a, tl, b, lo, hi);
+  const typename Rec<T>::V *rf = (const typename Rec<T>::V *)a.rfs + (size_t)b * a.nchrg;
+  const int2 *ri = a.ris + (size_t)b * a.nchrg;
   int org[3];
   tile_origin(a, tl, org[0], org[1], org[2]);
   const int H0 = a.H[0], H01 = a.H[0] * a.H[1];
@@ -214,12 +439,12 @@ __global__ void __launch_bounds__(spread_lanes<T>() * PME_BLOCK) k_pme_spread(Pm
   // (more wavefronts in flight for the LDS atomics)
   constexpr int L = spread_lanes<T>();
   const int part = tid % L;
-  for (int c = tid / L; c < cnt; c += blockDim.x / L) {
-    const int it = a.sorted[lo + c];
-    const T q = (T)a.q[a.ichrg[it % a.nchrg]];
+  for (int c = lo + tid / L; c < hi; c += blockDim.x / L) {
+    const typename Rec<T>::V f = rf[c];
+    const T q = f.w;
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, false, T>(a, it, org, w, dw, l);
+    item_weights<NI, false, T>(f, ri[c].x, org, w, dw, l);
 #pragma unroll
     for (int m = 0; m < NI; m++) w[0][m] *= q;
     for (int rw = part; rw < NI * NI; rw += L) {
@@ -292,9 +517,11 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
   int tl, b;
   xcd_unit_bead(a.ntile, a.P, tl, b);
   const int tid = threadIdx.x;
-  const size_t bin = (size_t)b * a.ntile + tl;
-  const int lo = a.bin_off[bin], cnt = a.bin_cnt[bin];
-  if (cnt == 0) return;  // uniform over the workgroup
+  int lo, hi_;
+  tile_items(a, tl, b, lo, hi_);
+  if (lo == hi_) return;  // uniform over the workgroup
+  const typename Rec<T>::V *rf = (const typename Rec<T>::V *)a.rfs + (size_t)b * a.nchrg;
+  const int2 *ri = a.ris + (size_t)b * a.nchrg;
   int org[3];
   tile_origin(a, tl, org[0], org[1], org[2]);
   const int Ka = a.K[0], Kb = a.K[1], Kc = a.K[2];
@@ -306,13 +533,12 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
   constexpr int HP = L == 1 ? 0 : NI / 2;  // planes of lane 0 when split
   constexpr int KP = NI - HP;              // planes per lane (lane 0 pads odd orders with zero weights)
   const int part = L == 1 ? 0 : (tid & 1);
-  for (int c = tid / L; c < cnt; c += blockDim.x / L) {
-    const int it = a.sorted[lo + c];
-    const int ic = it % a.nchrg, bead = it / a.nchrg;
-    const int i = a.ichrg[ic];
+  for (int c = lo + tid / L; c < hi_; c += blockDim.x / L) {
+    const int2 si = ri[c];
+    const int i = a.ichrg[si.y];
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, true, T>(a, it, org, w, dw, l);
+    item_weights<NI, true, T>(rf[c], si.x, org, w, dw, l);
     // this lane's planes: weights picked once per charge
     T w2[KP], dw2[KP];
 #pragma unroll
@@ -358,7 +584,7 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
       db *= (double)Kb * q;
       dc *= (double)Kc * q;
       // bead-major, so the lines of one bead are written from its own XCD
-      const size_t ib = (size_t)bead * a.N + i;
+      const size_t ib = (size_t)b * a.N + i;
       a.rx[ib] = -(da * hi[0] + db * hi[1] + dc * hi[2]);
       a.ry[ib] = -(da * hi[3] + db * hi[4] + dc * hi[5]);
       a.rz[ib] = -(da * hi[6] + db * hi[7] + dc * hi[8]);
@@ -377,21 +603,22 @@ __global__ void __launch_bounds__(PME_BLOCK) k_pme_phi(PmeArgs a) {
   int tl, b;
   xcd_unit_bead(a.ntile, a.P, tl, b);
   const int tid = threadIdx.x;
-  const size_t bin = (size_t)b * a.ntile + tl;
-  const int lo = a.bin_off[bin], cnt = a.bin_cnt[bin];
-  if (cnt == 0) return;  // uniform over the workgroup
+  int lo, hi_;
+  tile_items(a, tl, b, lo, hi_);
+  if (lo == hi_) return;  // uniform over the workgroup
+  const typename Rec<T>::V *rf = (const typename Rec<T>::V *)a.rfs + (size_t)b * a.nchrg;
+  const int2 *ri = a.ris + (size_t)b * a.nchrg;
   int org[3];
   tile_origin(a, tl, org[0], org[1], org[2]);
   const int H0 = a.H[0], H01 = H0 * a.H[1];
   load_halo<T>(a, b, org, box);
   __syncthreads();
-  for (int c = tid; c < cnt; c += blockDim.x) {
-    const int it = a.sorted[lo + c];
-    const int ic = it % a.nchrg, bead = it / a.nchrg;
-    const int i = a.ichrg[ic];
+  for (int c = lo + tid; c < hi_; c += blockDim.x) {
+    const int2 si = ri[c];
+    const int i = a.ichrg[si.y];
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, false, T>(a, it, org, w, dw, l);
+    item_weights<NI, false, T>(rf[c], si.x, org, w, dw, l);
     double v = 0.0;
     for (int mc = 0; mc < NI; mc++) {
 #pragma unroll
@@ -403,7 +630,7 @@ __global__ void __launch_bounds__(PME_BLOCK) k_pme_phi(PmeArgs a) {
         v += (double)(r * (w[1][mb] * w[2][mc]));
       }
     }
-    a.phi[(size_t)i * a.P + bead] += v;
+    a.phi[(size_t)i * a.P + b] += v;
   }
 }
 
@@ -417,6 +644,18 @@ size_t pme_lds_bytes(const PmeArgs &a, bool gather) {
 
 template <typename T>
 hipError_t launch_spread_t(const PmeArgs &a, hipStream_t st) {
+  if (a.mm) {
+    const dim3 g(xcd_grid(a.ntile, a.P));
+    switch (a.n) {
+      case 4: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_spread_mm<4, T>), g, dim3(64), 0, st, a); break;
+      case 5: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_spread_mm<5, T>), g, dim3(64), 0, st, a); break;
+      case 6: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_spread_mm<6, T>), g, dim3(64), 0, st, a); break;
+      case 7: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_spread_mm<7, T>), g, dim3(64), 0, st, a); break;
+      case 8: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_spread_mm<8, T>), g, dim3(64), 0, st, a); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   const dim3 grid(xcd_grid(a.ntile, a.P)), block(spread_lanes<T>() * PME_BLOCK);
   const size_t lds = pme_lds_bytes(a, false);
   switch (a.n) {

@@ -12,6 +12,13 @@ pytestmark = pytest.mark.gpu
 FP64_TOL = 1e-9
 
 
+@pytest.fixture(scope="module", autouse=True)
+def torch_first():
+    """torch finds the GPU only if it looks before the library does."""
+    import torch
+    torch.cuda.init()
+
+
 def call(c, **kw):
     from piny_amd.engine import Engine
     flags = abi.PMX_EVAL_PIMD if c.system.pi_beads > 1 else 0
@@ -126,3 +133,22 @@ def test_list_rows(monkeypatch, mode, nmol, P, cell):
     for a, b in zip(eng.verlet_list(), o.verlet_list()):
         assert np.array_equal(a, b)
     eng.close()
+
+
+# PME: a bead's sort in one workgroup and in three launches, the matrix-core
+# spread (10^5 items) and the LDS one, orders and grids with and without its
+# tiles, FP64 and mixed (the mixed bars of the parity tests)
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("nmol, P, order, kmax", [(64, 1, 4, 6), (690, 1, 6, 10), (530, 64, 6, 10), (530, 64, 4, 14),
+                                                  (530, 64, 8, 14), (600, 60, 7, 17), (90, 2, 9, 10),
+                                                  (530, 64, 5, 8)])
+def test_pme_bins_and_spread(prec, nmol, P, order, kmax):
+    c = w.small_config(w.SPC_FW, nmol=nmol, P=P, seed=nmol + order, cutoff=2.5, kmax=kmax)
+    c.system.settings.n_interp = order
+    if prec == "fp64":
+        return check(c)
+    e, f, eo, fo = call(c, precision=abi.PMX_PREC_MIXED)
+    scale = max(abs(eo[k]) for k in abi.ENERGY_KEYS)
+    for k in abi.ENERGY_KEYS:
+        assert abs(e[k] - eo[k]) < 1e-5 * scale, k
+    assert np.sqrt(((f - fo) ** 2).sum() / (fo ** 2).sum()) < 1e-4
