@@ -366,7 +366,11 @@ void auto_tile_caps(const Setup &s, int n, int cap[3]) {
       if (K % t == 0) return t;
     return 0;
   };
-  const int lo = n - 1, t0 = divisor(s.ngrid[0], lo, 17 - n), t1 = divisor(s.ngrid[1], lo, 17 - n);
+  const int lo = n - 1, t1 = divisor(s.ngrid[1], lo, 17 - n);
+  // along a a multiple of 4, which the gather loads 16 bytes at a time, where there is one
+  int t0 = divisor(s.ngrid[0], lo, 17 - n);
+  for (int t = (17 - n) & ~3; t >= lo && t0 % 4; t -= 4)
+    if (s.ngrid[0] % t == 0) t0 = t;
   int t2 = divisor(s.ngrid[2], lo, (long)s.P * (long)s.ichrg.size() >= PME_MM_ITEMS ? 12 : std::max(lo, 8));
   cap[0] = cap[1] = 16;
   cap[2] = 8;

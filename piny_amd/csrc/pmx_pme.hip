@@ -499,19 +499,59 @@ __device__ __forceinline__ void load_halo(const PmeArgs &a, int b, const int (&o
   }
 }
 
-// lanes per charge in the gather: with FP32 grids two, each summing half
-// of the support planes (twice the wavefronts on the LDS the halo box
-// allows); with FP64 one
+// The same box by rows of 16 points, V of them a lane (8 or 16 bytes), for
+// tiles whose first point is V-aligned in the grid (T[0] a multiple of V, so
+// the grid's rows are too) and whose rows are at most 16 wide: the lane's
+// column, its wrap included, is fixed, and only the row is divided into (b, c)
+// and wrapped.  One point a lane took some 22 instructions each, half of the
+// gather's.  The points past the row's end are read (they lie in the grid) and
+// stored in the row's padding; rows are box_stride apart, which keeps the
+// vector stores aligned and lets neighbouring rows start on other banks (at a
+// stride of 16 the gather's reads met on them: FP64 68 us).
 template <typename T>
-constexpr int gather_lanes() {
-  return sizeof(T) == 4 ? 2 : 1;
+__host__ __device__ constexpr int box_stride() {
+  return sizeof(T) == 4 ? 20 : 18;
+}
+template <typename T, int V>
+__device__ __forceinline__ void load_halo_rows(const PmeArgs &a, int b, const int (&org)[3], T *box) {
+  typedef T vec __attribute__((ext_vector_type(V)));
+  constexpr int LR = 16 / V;  // lanes per row
+  const int Ka = a.K[0], Kb = a.K[1], Kc = a.K[2], H1 = a.H[1], rows = H1 * a.H[2];
+  const T *g = (const T *)a.grid + (size_t)b * a.gstride;
+  const int q = threadIdx.x % LR, step = blockDim.x / LR;
+  int ga = org[0] + q * V;
+  while (ga >= Ka) ga -= Ka;
+  for (int r0 = threadIdx.x / LR; r0 < rows; r0 += 4 * step) {
+    vec v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int r = min(r0 + u * step, rows - 1), lc = (int)__umulhi((unsigned)r, a.mH1), lb = r - lc * H1;
+      // n - 1 <= K on every grid: two conditional subtractions wrap
+      int gb = org[1] + lb, gc = org[2] + lc;
+      gb -= gb >= Kb ? Kb : 0;
+      gc -= gc >= Kc ? Kc : 0;
+      gb -= gb >= Kb ? Kb : 0;
+      gc -= gc >= Kc ? Kc : 0;
+      v[u] = *(const vec *)(g + (gc * Kb + gb) * Ka + ga);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int r = r0 + u * step;
+      if (r < rows) *(vec *)(box + r * box_stride<T>() + q * V) = v[u];
+    }
+  }
 }
 
-// one workgroup per (tile, bead): the potential on the halo box into LDS,
-// then L lanes per charge (ewald3d_pme.c:534-560); lane part sums the planes
-// mc = part * NI / 2 ... (part + 1) * NI / 2 - 1 and the pair adds its sums
-template <int NI, typename T>
-__global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(PmeArgs a) {
+// One workgroup per (tile, bead): the potential on the halo box into LDS,
+// then two lanes per charge (ewald3d_pme.c:534-560); lane part sums the planes
+// mc = part * NI / 2 ... and the pair adds its sums.  Row sums in T; their
+// products with the other axes' weights and the sums over rows in FP64.  V:
+// points a lane loads (load_halo_rows), 0 for tiles it does not take.
+// 4096 q-TIP4P/F at P = 32, mixed 35 -> 26 us, FP64 47 -> 40 us (its LDS
+// reads are three quarters of that, the other half of the bank conflicts being
+// the charges' random places).
+template <int NI, typename T, int V>
+__global__ void __launch_bounds__(256) k_pme_gather(PmeArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T *box = (T *)lds_raw;
   int tl, b;
@@ -525,42 +565,39 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
   int org[3];
   tile_origin(a, tl, org[0], org[1], org[2]);
   const int Ka = a.K[0], Kb = a.K[1], Kc = a.K[2];
-  const int H0 = a.H[0], H01 = H0 * a.H[1];
-  load_halo<T>(a, b, org, box);
+  const int H0 = V > 0 ? box_stride<T>() : a.H[0], H01 = H0 * a.H[1];
+  if constexpr (V > 0) load_halo_rows<T, V>(a, b, org, box);
+  else load_halo<T>(a, b, org, box);
   __syncthreads();
   const double *hi = a.cell.hi;
-  constexpr int L = gather_lanes<T>();
-  constexpr int HP = L == 1 ? 0 : NI / 2;  // planes of lane 0 when split
-  constexpr int KP = NI - HP;              // planes per lane (lane 0 pads odd orders with zero weights)
-  const int part = L == 1 ? 0 : (tid & 1);
-  for (int c = lo + tid / L; c < hi_; c += blockDim.x / L) {
+  constexpr int HP = NI / 2;   // planes of lane 0
+  constexpr int KP = NI - HP;  // planes per lane (lane 0 pads odd orders with zero weights)
+  const int part = tid & 1;
+  for (int c = lo + tid / 2; c < hi_; c += blockDim.x / 2) {
     const int2 si = ri[c];
+    const typename Rec<T>::V f = rf[c];
     const int i = a.ichrg[si.y];
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, true, T>(rf[c], si.x, org, w, dw, l);
-    // this lane's planes: weights picked once per charge
-    T w2[KP], dw2[KP];
+    item_weights<NI, true, T>(f, si.x, org, w, dw, l);
+    double wb[NI], dwb[NI];
 #pragma unroll
-    for (int k = 0; k < KP; k++) {
-      if (L == 1) {
-        w2[k] = w[2][k];
-        dw2[k] = dw[2][k];
-      } else {
-        const T a0 = k < HP ? w[2][k] : (T)0, d0 = k < HP ? dw[2][k] : (T)0;
-        w2[k] = part ? w[2][HP + k] : a0;
-        dw2[k] = part ? dw[2][HP + k] : d0;
-      }
+    for (int m = 0; m < NI; m++) {
+      wb[m] = (double)w[1][m];
+      dwb[m] = (double)dw[1][m];
     }
-    const int mc0 = part * HP;
-    // row sums in T, accumulated over rows in FP64
+    const T *base = box + (l[2] + part * HP) * H01 + l[1] * H0 + l[0];
     double da = 0.0, db = 0.0, dc = 0.0;
 #pragma unroll
     for (int k = 0; k < KP; k++) {
-      const int mc = min(mc0 + k, NI - 1);
+      // lane 0 has HP planes: with an odd order its last is lane 1's first,
+      // with weight zero
+      const T a0 = k < HP ? w[2][k] : (T)0, d0 = k < HP ? dw[2][k] : (T)0;
+      const double wc = (double)(part ? w[2][HP + k] : a0), dwc = (double)(part ? dw[2][HP + k] : d0);
+      double pa = 0.0, pb = 0.0, pc = 0.0;
 #pragma unroll
       for (int mb = 0; mb < NI; mb++) {
-        const T *row = box + (l[2] + mc) * H01 + (l[1] + mb) * H0 + l[0];
+        const T *row = base + mb * H0;
         T r0 = (T)0, r1 = (T)0;
 #pragma unroll
         for (int ma = 0; ma < NI; ma++) {
@@ -568,16 +605,19 @@ __global__ void __launch_bounds__(gather_lanes<T>() * PME_BLOCK) k_pme_gather(Pm
           r0 += dw[0][ma] * phi;
           r1 += w[0][ma] * phi;
         }
-        da += (double)(r0 * (w[1][mb] * w2[k]));
-        db += (double)(r1 * (dw[1][mb] * w2[k]));
-        dc += (double)(r1 * (w[1][mb] * dw2[k]));
+        pa += (double)r0 * wb[mb];
+        pb += (double)r1 * dwb[mb];
+        pc += (double)r1 * wb[mb];
       }
+      da += pa * wc;
+      db += pb * wc;
+      dc += pc * dwc;
+      base += H01;
     }
-    if (L == 2) {  // the pair's lanes hold the same charge
-      da += __shfl_xor(da, 1, 64);
-      db += __shfl_xor(db, 1, 64);
-      dc += __shfl_xor(dc, 1, 64);
-    }
+    // the pair's lanes hold the same charge
+    da = dpp_rotate_add<0xB1>(da);  // quad_perm 1, 0, 3, 2
+    db = dpp_rotate_add<0xB1>(db);
+    dc = dpp_rotate_add<0xB1>(dc);
     if (part == 0) {
       const double q = a.q[i];
       da *= (double)Ka * q;
@@ -672,16 +712,28 @@ hipError_t launch_spread_t(const PmeArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int NI, typename T, int V>
+void launch_gather_v(const PmeArgs &a, hipStream_t st) {
+  const size_t lds = V > 0 ? (size_t)box_stride<T>() * a.H[1] * a.H[2] * sizeof(T) : pme_lds_bytes(a, true);
+  if (lds > 65536)
+    (void)hipFuncSetAttribute((const void *)k_pme_gather<NI, T, V>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  // two lanes per charge: 256 lanes when a tile holds over 64 charges on average
+  const int lanes = (long)a.nchrg > 64l * a.ntile ? 256 : 128;
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_gather<NI, T, V>), dim3(xcd_grid(a.ntile, a.P)), dim3(lanes), lds, st, a);
+}
+
 template <typename T>
 hipError_t launch_gather_t(const PmeArgs &a, hipStream_t st) {
-  const dim3 grid(xcd_grid(a.ntile, a.P)), block(gather_lanes<T>() * PME_BLOCK);
-  const size_t lds = pme_lds_bytes(a, true);
+  constexpr int V2 = 16 / (int)sizeof(T), V1 = V2 / 2;  // points of a 16 and an 8 byte load
+  // rows of up to 16 points; their padding must fit the LDS where the box does
+  const bool rows = a.H[0] <= 16 && (size_t)box_stride<T>() * a.H[1] * a.H[2] * sizeof(T) <= FFT_LDS_MAX;
+  const int v = !rows ? 0 : a.T[0] % V2 == 0 ? V2 : a.T[0] % V1 == 0 ? V1 : 0;
   switch (a.n) {
-#define X(NI) \
-  case NI:                                                                                                  \
-    if (lds > 65536)                                                                                          \
-      (void)hipFuncSetAttribute((const void *)k_pme_gather<NI, T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_pme_gather<NI, T>), grid, block, lds, st, a);                                \
+#define X(NI)                                                    \
+  case NI:                                                       \
+    if (v == V2) launch_gather_v<NI, T, V2>(a, st);              \
+    else if (v == V1) launch_gather_v<NI, T, V1>(a, st);         \
+    else launch_gather_v<NI, T, 0>(a, st);                       \
     break;
     PMX_PME_CASES(X)
 #undef X
