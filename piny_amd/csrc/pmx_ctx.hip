@@ -1625,7 +1625,7 @@ int launch_pme(pmx_ctx *c, hipStream_t sk) {
   f.mKa = (unsigned)((1ull << 32) / (unsigned)s.ngrid[0] + 1ull);
   f.mT0 = a.mT0;
   f.mT1 = a.mT1;
-  HIPCHK(launch_pme_fft(f, sk));
+  HIPCHK(f.f32 ? launch_pme_fft32(f, sk) : launch_pme_fft64(f, sk));
   HIPCHK(launch_pme_gather(a, sk));
   return PMX_OK;
 }

@@ -488,7 +488,9 @@ hipError_t launch_pme_spread(const PmeArgs &a, hipStream_t st);
 hipError_t launch_pme_gather(const PmeArgs &a, hipStream_t st);
 hipError_t launch_pme_phi(const PmeArgs &a, hipStream_t st);
 hipError_t launch_ewald(const EwaldArgs &a, hipStream_t st);
-hipError_t launch_pme_fft(const FftArgs &f, hipStream_t st);
+// forward 3-D FFT, convolution with energy and virial, inverse 3-D FFT of FP32 and FP64 grids
+hipError_t launch_pme_fft32(const FftArgs &f, hipStream_t st);
+hipError_t launch_pme_fft64(const FftArgs &f, hipStream_t st);
 // block size for grid-stride kernels whose threads keep one bead: the
 // largest multiple of P not above 256
 inline int bead_block(int P) { return 256 - (256 % P); }

@@ -152,3 +152,21 @@ def test_pme_bins_and_spread(prec, nmol, P, order, kmax):
     for k in abi.ENERGY_KEYS:
         assert abs(e[k] - eo[k]) < 1e-5 * scale, k
     assert np.sqrt(((f - fo) ** 2).sum() / (fo ** 2).sum()) < 1e-4
+
+
+# every grid size with FFT kernels of its own, and one without (100), against
+# the oracle's own transform of the same grid
+@pytest.mark.parametrize("K", [12, 16, 20, 24, 32, 36, 40, 48, 60, 64, 72, 80, 96, 100])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_fft_sizes(prec, K):
+    if prec == "fp64" and K == 100:
+        pytest.skip("a 100 x 100 FP64 plane and its twiddles exceed a workgroup's LDS")
+    c = w.small_config(w.SPC_FW, nmol=64, P=2, seed=K, kmax=2 * (K // 4 - 1))
+    c.system.settings.kmax_ewd = min(c.system.settings.kmax_ewd, K // 2 - 2)
+    if prec == "fp64":
+        check(c)
+    else:
+        e, f, eo, fo = call(c, precision=abi.PMX_PREC_MIXED)
+        scale = max(abs(eo[k]) for k in abi.ENERGY_KEYS)
+        assert abs(e["vrecip"] - eo["vrecip"]) < 1e-5 * scale
+        assert np.sqrt(((f - fo) ** 2).sum() / (fo ** 2).sum()) < 1e-4
