@@ -168,7 +168,7 @@ struct pmx_ctx {
   int overlap = 0;
   bool last_overlap = false;  // the last force sequence ran PME on sk
   bool pme_deferred = false;  // PME on sk still to be launched, by main_sequence after the pair kernel
-  bool fuse_pack = false;     // k_list_check writes site, disp and umax (mixed precision, P a power of 2 <= 64)
+  bool fuse_pack = false;     // k_list_check writes site, disp and umax (P a power of 2, 2 to 64)
   hipStream_t sk = nullptr;
   hipEvent_t kfork = nullptr, kjoin = nullptr;
   hipEvent_t mxev = nullptr;  // the list check's maxima are in mx_pin
@@ -1046,10 +1046,12 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
         return PMX_ERR_RANGE;
       }
       TRY(dalloc(c, &c->disp, NP));
-      c->fuse_pack = P <= 64 && (64 % P) == 0;  // the list check packs the sites and displacements
     }
     if (c->pair_mode == 2) TRY(build_pair_tables(c));
     if (P > 1) TRY(dalloc(c, &c->umax, (size_t)N));
+    // with beads the list check packs the sites, their largest displacements
+    // and (mixed) the displacements
+    c->fuse_pack = P > 1 && P <= 64 && (64 % P) == 0;
   }
   TRY(dalloc(c, &c->site_cell, N));
   TRY(dalloc(c, &c->site_pos, N));
@@ -1511,6 +1513,17 @@ bool clu_active(const pmx_ctx *c) { return c->clu_on && !respa_on(c); }
 
 namespace {
 
+// The site records of a one-bead context hold its charges alone (the pair
+// kernels read positions): packed when the charges are set, not on each call.
+int pack_charges(pmx_ctx *c) {
+  if (c->s.P > 1) return PMX_OK;
+  hipLaunchKernelGGL(k_pack_sites, dim3(blocks(c->s.N)), dim3(256), 0, c->st, c->s.N, 0, c->xm, c->ym, c->zm, c->q,
+                     c->site);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(c->st));
+  return PMX_OK;
+}
+
 // How the list check sets xmod: 0 given (or no beads), 1 the bead centroid
 // (normal modes), 2 bead 1 (staging): mode 1 of the transform, which
 // control_pimd_trans_pos copies into xmod (control_pimd_trans.c:175-181).
@@ -1655,7 +1668,7 @@ int pre_sequence(pmx_ctx *c, unsigned flags, hipStream_t st, bool timing, bool f
   // with fuse_pack the list check has packed the sites and displacements
   // (list_stage_launch precedes every force sequence; a weighted call's
   // second pass reuses the first pass's, the positions being the same)
-  if (!c->fuse_pack) {
+  if (!c->fuse_pack && P > 1) {  // of one bead the records are the charges (pack_charges)
     hipLaunchKernelGGL(k_pack_sites, dim3(blocks(N)), dim3(256), 0, st, N, P > 1 ? 1 : 0, c->xm, c->ym, c->zm,
                        c->q, c->site);
     HIPCHK(hipGetLastError());
@@ -1673,7 +1686,7 @@ int pre_sequence(pmx_ctx *c, unsigned flags, hipStream_t st, bool timing, bool f
       hipLaunchKernelGGL(k_site_umax, dim3(blocks(N)), dim3(256), 0, st, N, P, c->disp, c->umax);
     }
     HIPCHK(hipGetLastError());
-  } else if (!c->disp && c->umax && c->full_list) {
+  } else if (!c->disp && c->umax && c->full_list && !c->fuse_pack) {
     hipLaunchKernelGGL(k_site_umax64, dim3(blocks(N)), dim3(256), 0, st, N, P, c->x, c->y, c->z, c->xm, c->ym,
                        c->zm, c->umax);
     HIPCHK(hipGetLastError());
@@ -2218,6 +2231,11 @@ pmx_ctx *pmx_create(const pmx_system *sys, const pmx_params *par, const double *
   if (const char *env = getenv("PMX_PME_TILE"))  // tuning override "Ta,Tb,Tc" (upper bounds)
     sscanf(env, "%d,%d,%d", &c->tile_cap[0], &c->tile_cap[1], &c->tile_cap[2]);
   if (build_device(c, sys) != PMX_OK) {
+    std::string e = c->err;
+    pmx_destroy(c);
+    return fail("pmx_create: " + e);
+  }
+  if (pack_charges(c) != PMX_OK) {
     std::string e = c->err;
     pmx_destroy(c);
     return fail("pmx_create: " + e);
@@ -3279,6 +3297,7 @@ int pmx_set_force_field(pmx_ctx *c, const pmx_system *sys) {
   HIPCHK(hipStreamSynchronize(c->st));
   const size_t N = (size_t)s.N;
   HIPCHK(hipMemcpy(c->q, sys->q, N * sizeof(double), hipMemcpyHostToDevice));
+  if (int rc = pack_charges(c)) return rc;
   if (int rc = setup_molecules(c, sys)) return rc;  // the templates hold charge products
   {
     const size_t nt = (size_t)s.npair * s.nsplin;

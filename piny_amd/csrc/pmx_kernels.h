@@ -371,8 +371,9 @@ __global__ void k_pack_disp_umax(int N, int P, const double *x, const double *y,
                                  const double *ym, const double *zm, float4 *u, double *umax);
 __global__ void k_site_umax64(int N, int P, const double *x, const double *y, const double *z, const double *xm,
                               const double *ym, const double *zm, double *umax);
-// Pack: what k_pack_sites and k_pack_disp_umax write, formed in the same
-// pass (disp non-null: mixed precision with P a power of two up to 64).
+// Pack (site non-null: beads, P a power of two up to 64): what k_pack_sites
+// and, with disp (mixed precision), k_pack_disp_umax or, without, k_site_umax64
+// write, formed in the same pass.
 struct CheckPack {
   float4 *disp;
   double *umax;

@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(256) k_list_check(int N, int P, const double *
         zm[i] = zi;
       }
     }
-    if (pk.disp) {  // uniform; P divides 64, so the site's beads are this group's lanes
+    if (pk.site) {  // uniform; P divides 64, so the site's beads are this group's lanes
       // the site's xmod as the lead lane has it (formed above, or given)
       double rx = 0.0, ry = 0.0, rz = 0.0;
       if (act && k == 0) {
@@ -334,16 +334,26 @@ __global__ void __launch_bounds__(256) k_list_check(int N, int P, const double *
       rx = shfl_d(rx, lead);
       ry = shfl_d(ry, lead);
       rz = shfl_d(rz, lead);
-      // k_pack_disp_umax and k_pack_sites
-      float m = 0.0f;
-      if (act) {
-        const float4 v = make_float4((float)(xk - rx), (float)(yk - ry), (float)(zk - rz), 0.0f);
-        pk.disp[base + k] = v;
-        m = v.x * v.x + v.y * v.y + v.z * v.z;
+      // k_pack_disp_umax (mixed) or k_site_umax64, and k_pack_sites
+      double um = 0.0;
+      if (pk.disp) {
+        float m = 0.0f;
+        if (act) {
+          const float4 v = make_float4((float)(xk - rx), (float)(yk - ry), (float)(zk - rz), 0.0f);
+          pk.disp[base + k] = v;
+          m = v.x * v.x + v.y * v.y + v.z * v.z;
+        }
+        for (int off = 1; off < G; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        um = (double)m;
+      } else {
+        if (act) {
+          const double dx = xk - rx, dy = yk - ry, dz = zk - rz;
+          um = dx * dx + dy * dy + dz * dz;
+        }
+        for (int off = 1; off < G; off <<= 1) um = fmax(um, __shfl_xor(um, off, 64));
       }
-      for (int off = 1; off < G; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
       if (act && k == 0) {
-        pk.umax[i] = sqrt((double)m);
+        pk.umax[i] = sqrt(um);
         pk.site[i] = make_double4(rx, ry, rz, pk.q[i]);
       }
     }
