@@ -1191,7 +1191,8 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
     TRY(setup_pme_tiles(c));
   }
   {
-    const size_t pair = (size_t)pair_grid_x(N, PAIR_MAX_WAVES) * P * PAIR_NV;
+    const size_t pair =
+        (size_t)std::max(pair_grid_x(N, PAIR_MAX_WAVES), pair_tab_grid_x(N, PAIR_MAX_WAVES)) * P * PAIR_NV;
     const size_t fft = (size_t)std::max(c->pme ? s.ngrid[1] : 0,
                                         c->ewald ? (s.nktot + EWALD_BLOCK - 1) / EWALD_BLOCK : 0) *
                        P * FFT_NV;

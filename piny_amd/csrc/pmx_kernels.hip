@@ -1607,7 +1607,7 @@ __global__ void __launch_bounds__(64 * TAB_WAVES) k_pair_tab_lds(PairArgs a) {
   int npr = 0;
   const int spb = TAB_WAVES / W;  // sites per workgroup and round
   for (int i0 = blockIdx.x * spb; i0 < a.N; i0 += gridDim.x * spb) {
-    const int i = i0 + w / W;
+    const int i = w < spb * W ? i0 + w / W : a.N;  // 16 wavefronts in spb groups of W, the rest idle
     const size_t ib = (size_t)min(i, a.N - 1) * P + (bact ? bead : 0);
     double fxi = 0.0, fyi = 0.0, fzi = 0.0;
     if (i < a.N) {
@@ -1733,7 +1733,7 @@ __global__ void __launch_bounds__(64 * TAB_WAVES) k_pair_tab_lds(PairArgs a) {
         sf[128 + lane] = fzi;
       }
       __syncthreads();
-      if (part == 0 && slot == 0)
+      if (part == 0 && slot == 0 && i < a.N)
         for (int q = 1; q < W; q++) {
           const double *so = (const double *)sdf[w + q];
           fxi += so[lane];
@@ -3026,13 +3026,23 @@ bool pair_tab_lds_fits(int nsplin) {
   return nsplin >= 512 && (size_t)nsplin * sizeof(double2) + 50 * 1024 <= FFT_LDS_MAX;
 }
 int pair_tab_wps(int N) {
-  int W = 1;
-  while (W < 4 && N * W * 2 <= 4096) W *= 2;
-  return W;
+  // rounds of the 256 workgroups the chip holds, times the chunks of a row
+  // (some six) that one of its wavefronts takes: 343 SPC/Fw at P = 16 (1029
+  // sites) take 56 us with two wavefronts a site (129 workgroups) and 43 us
+  // with three (206), where four would be 258 workgroups and a second round
+  int best = 1, cost = 1 << 30;
+  for (int W : {1, 2, 3, 4, 6}) {
+    const int spb = TAB_WAVES / W, groups = (N + spb - 1) / spb, c = (groups + 255) / 256 * ((6 + W - 1) / W);
+    if (c < cost) {
+      cost = c;
+      best = W;
+    }
+  }
+  return best;
 }
 int pair_tab_grid_x(int N, int max_waves) {
-  const int sites = std::min(N, max_waves), W = pair_tab_wps(N);
-  return std::max(1, (sites * W + TAB_WAVES - 1) / TAB_WAVES);
+  const int spb = TAB_WAVES / pair_tab_wps(N);
+  return std::max(1, std::min((N + spb - 1) / spb, max_waves / TAB_WAVES));
 }
 
 // k_pair_mixed with the erfc term formed as TM says, with or without beads

@@ -75,7 +75,8 @@ def test_positions_in_and_out(nmol, P):
 
 # the FP64 table kernel: wavefronts sharing a site (few sites), a partial last
 # workgroup, more sites than wavefronts, tables too short and too long for LDS
-@pytest.mark.parametrize("nmol, P, nsplin", [(27, 1, 5000), (201, 2, 5000), (343, 1, 512), (700, 1, 511),
+@pytest.mark.parametrize("nmol, P, nsplin", [(2, 1, 5000), (27, 1, 5000), (201, 2, 5000), (300, 2, 5000), (400, 4, 5000),
+                                             (430, 1, 5000), (343, 1, 512), (700, 1, 511),
                                              (1400, 1, 5000), (64, 8, 7200), (64, 8, 6900)])
 def test_pair_table_in_lds(nmol, P, nsplin):
     c = w.small_config(w.SPC_FW, nmol=nmol, P=P, seed=nmol)
