@@ -2921,6 +2921,24 @@ int pmx_get_positions(pmx_ctx *c, double *x, double *y, double *z) {
   return get_bead_major(c, src, x, y, z);
 }
 
+namespace {
+
+// One force call of an integrator's step, launched on the context's stream
+// without the readback of the energies (the list decision is the host's one
+// wait).
+int step_force(pmx_ctx *c, unsigned flags) {
+  pmx_energies tmp;
+  memset(&tmp, 0, sizeof tmp);
+  c->grad_ready = false;
+  if (int rc = list_stage_launch(c, c->st, false)) return rc;
+  if (int rc = pre_sequence(c, flags, c->st, false, true)) return rc;
+  HIPCHK(hipEventSynchronize(c->mxev));
+  if (int rc = list_stage_finish(c, flags, &tmp)) return rc;
+  return main_sequence(c, flags, c->st, false);
+}
+
+}  // namespace
+
 // Velocity Verlet in the NVE ensemble, int_NVE (md/int_NVE.c:29-125):
 // int_0_to_dt2_nve (int_0_to_dt2.c:35-124: v += f dt/2 / m, x += v dt, ghost
 // positions), the force call, int_dt2_to_dt_nve (int_dt2_to_dt.c:33-100:
@@ -2940,6 +2958,7 @@ int pmx_md_nve(pmx_ctx *c, int nsteps, double dt, pmx_energies *out, double *kin
     set_err(c, "pmx_md_nve: no positions set");
     return PMX_ERR_STATE;
   }
+  HIPCHK(hipSetDevice(c->device));
   const size_t N = (size_t)s.N;
   int rc = PMX_OK;
   if (!c->forces_valid || c->last_modes) {
@@ -2948,19 +2967,20 @@ int pmx_md_nve(pmx_ctx *c, int nsteps, double dt, pmx_energies *out, double *kin
   }
   const double dt2 = dt / 2.0;
   for (int step = 0; step < nsteps; step++) {
-    hipLaunchKernelGGL(k_vv_kick, dim3(blocks(N)), dim3(256), 0, c->st, (int)N, dt2, c->mass, c->fx, c->fy, c->fz,
-                       c->vx, c->vy, c->vz);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_vv_drift, dim3(blocks(N)), dim3(256), 0, c->st, (int)N, dt, c->vx, c->vy, c->vz, c->x,
-                       c->y, c->z);
+    hipLaunchKernelGGL(k_vv_move, dim3(blocks(N)), dim3(256), 0, c->st, (int)N, step > 0 ? 1 : 0, dt2, dt, c->mass,
+                       c->fx, c->fy, c->fz, c->vx, c->vy, c->vz, c->x, c->y, c->z);
     HIPCHK(hipGetLastError());
     if (c->nghost) {
       hipLaunchKernelGGL(k_ghost_pos, dim3(blocks((size_t)c->nghost)), dim3(256), 0, c->st, c->nghost, 1, c->gatom,
                          c->gncomp, c->gcomp, c->gcoef, c->x, c->y, c->z);
       HIPCHK(hipGetLastError());
     }
-    rc = pmx_energy_control(c, 0, out);
+    // only the last step's energies are returned: the others are not read
+    // back, except under the cluster kernel, whose check comes with them
+    rc = step + 1 < nsteps && !c->clu_enabled ? step_force(c, 0) : pmx_energy_control(c, 0, out);
     if (rc) return rc;
+  }
+  if (nsteps > 0) {
     hipLaunchKernelGGL(k_vv_kick, dim3(blocks(N)), dim3(256), 0, c->st, (int)N, dt2, c->mass, c->fx, c->fy, c->fz,
                        c->vx, c->vy, c->vz);
     HIPCHK(hipGetLastError());
@@ -3108,20 +3128,6 @@ int check_nhc_params(pmx_ctx *c, const pmx_nhc_params *np) {
   return PMX_OK;
 }
 
-// One force call of energy_control_pimd with mode forces, launched on the
-// context's stream without the readback of the energies (the list decision
-// is the host's one wait).
-int pimd_force(pmx_ctx *c, unsigned flags) {
-  pmx_energies tmp;
-  memset(&tmp, 0, sizeof tmp);
-  c->grad_ready = false;
-  if (int rc = list_stage_launch(c, c->st, false)) return rc;
-  if (int rc = pre_sequence(c, flags, c->st, false, true)) return rc;
-  HIPCHK(hipEventSynchronize(c->mxev));
-  if (int rc = list_stage_finish(c, flags, &tmp)) return rc;
-  return main_sequence(c, flags, c->st, false);
-}
-
 }  // namespace
 
 int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies *out, double *econs) {
@@ -3153,7 +3159,7 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
   memset(out, 0, sizeof(*out));
   // forces at the starting positions, xmod as the context has it
   if (c->clu_ok) hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->st, c->clu_flag + 1, 0, (size_t)1);
-  if (int rc = pimd_force(c, flags)) return rc;
+  if (int rc = step_force(c, flags)) return rc;
   const bool xmod_given = c->xmod_given;
   c->xmod_given = true;  // xmod is mode 1 of each drift from here on
   const unsigned gN = blocks(N);
@@ -3170,7 +3176,7 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
       rc = PMX_ERR_DEVICE;
       break;
     }
-    if ((rc = pimd_force(c, flags))) break;
+    if ((rc = step_force(c, flags))) break;
     (void)launch_nhc(a, NHC_KICK1, 0, c->st);
     hipLaunchKernelGGL(k_nhc_ckin, dim3(NHC_BLOCKS), dim3(256), 0, c->st, a);
     (void)launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);

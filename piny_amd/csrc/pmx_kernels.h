@@ -415,8 +415,9 @@ __global__ void k_ghost_force(int ng, int P, const int *gatom, const int *gncomp
 hipError_t launch_mode_forces(const ModeArgs &a, hipStream_t st);
 __global__ void k_vv_kick(int n, double dt2, const double *mass, const double *fx, const double *fy,
                           const double *fz, double *vx, double *vy, double *vz);
-__global__ void k_vv_drift(int n, double dt, const double *vx, const double *vy, const double *vz, double *x,
-                           double *y, double *z);
+__global__ void k_vv_move(int n, int ends, double dt2, double dt, const double *mass, const double *fx,
+                          const double *fy, const double *fz, double *vx, double *vy, double *vz, double *x, double *y,
+                          double *z);
 __global__ void k_kinetic(int n, const double *mass, const double *vx, const double *vy, const double *vz,
                           double *ke);
 

@@ -2544,14 +2544,31 @@ __global__ void k_vv_kick(int n, double dt2, const double *__restrict__ mass, co
   vz[i] += fz[i] * dt2 / m;
 }
 
-__global__ void k_vv_drift(int n, double dt, const double *__restrict__ vx, const double *__restrict__ vy,
-                           const double *__restrict__ vz, double *x, double *y, double *z) {
+// One velocity-Verlet move between two force calls: the second half kick of
+// the step that ends (when there is one), the first of the next, and its drift.
+__global__ void k_vv_move(int n, int ends, double dt2, double dt, const double *__restrict__ mass,
+                          const double *__restrict__ fx, const double *__restrict__ fy,
+                          const double *__restrict__ fz, double *vx, double *vy, double *vz, double *x, double *y,
+                          double *z) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  x[i] += vx[i] * dt;
-  y[i] += vy[i] * dt;
-  z[i] += vz[i] * dt;
+  const double m = mass[i], kx = fx[i] * dt2 / m, ky = fy[i] * dt2 / m, kz = fz[i] * dt2 / m;
+  double ux = vx[i], uy = vy[i], uz = vz[i];
+  if (ends) {
+    ux += kx;
+    uy += ky;
+    uz += kz;
+  }
+  ux += kx;
+  uy += ky;
+  uz += kz;
+  vx[i] = ux;
+  vy[i] = uy;
+  vz[i] = uz;
+  x[i] += ux * dt;
+  y[i] += uy * dt;
+  z[i] += uz * dt;
 }
 
 // kinetic energy 1/2 sum m v^2 (get_tvten), one atomic per wavefront
