@@ -165,7 +165,7 @@ struct pmx_ctx {
   hipEvent_t ready = nullptr;  // list stage done (batched calls)
   // PME on a second stream, concurrent with the pair kernel (the pair
   // kernel is bound by vector ALU issue, PME by memory and LDS)
-  int overlap = 0;
+  int overlap = 0;           // PME on sk beside the pair kernel (pmx_create's rule, or the autotuner)
   bool last_overlap = false;  // the last force sequence ran PME on sk
   bool pme_deferred = false;  // PME on sk still to be launched, by main_sequence after the pair kernel
   bool fuse_pack = false;     // k_list_check writes site, disp and umax (P a power of 2, 2 to 64)
@@ -2223,7 +2223,6 @@ pmx_ctx *pmx_create(const pmx_system *sys, const pmx_params *par, const double *
     pmx_destroy(c);
     return fail("pmx_create: stream creation failed");
   }
-  if (const char *env = getenv("PMX_OVERLAP")) c->overlap = atoi(env) != 0;  // tuning override 0 / 1
   // tuning override: 1 runs the molecule-cluster form of the mixed pair
   // kernel where the box qualifies (the per-site form is the default)
   if (const char *env = getenv("PMX_CLUSTER")) c->clu_enabled = atoi(env) == 1;
@@ -2236,6 +2235,15 @@ pmx_ctx *pmx_create(const pmx_system *sys, const pmx_params *par, const double *
     pmx_destroy(c);
     return fail("pmx_create: " + e);
   }
+  // PME beside the pair kernel on a stream of its own, where both are long:
+  // in mixed precision the pair kernel is bound by vector instructions, the
+  // k space by LDS, memory and the matrix cores, and from some 60000 (site,
+  // bead) on the pair gains more than the second stream's events cost (serial
+  // and beside: 179 and 198 us at 14400, 217 and 192 at 65536, 246 and 235 at
+  // 96000, 548 and 533 at 524288, 749 and 688 at 576048).  In FP64 the pair
+  // kernel's table fills a CU's LDS and registers, and nothing runs beside it.
+  c->overlap = c->pme && c->par.precision == PMX_PREC_MIXED && (size_t)c->s.N * c->s.P >= OVERLAP_ITEMS;
+  if (const char *env = getenv("PMX_OVERLAP")) c->overlap = atoi(env) != 0;  // tuning override 0 / 1
   if (pack_charges(c) != PMX_OK) {
     std::string e = c->err;
     pmx_destroy(c);

@@ -164,6 +164,7 @@ constexpr int EWALD_BLOCK = 256;
 
 constexpr int PME_NBIN_MAX = 1 << 17;  // bins of one bead
 constexpr long PME_MM_ITEMS = 100000;  // (charge, bead) items from which the matrix-core spread pays
+constexpr size_t OVERLAP_ITEMS = 60000;  // (site, bead) from which PME runs beside the mixed pair kernel
 constexpr int PME_ZB_MAX = 63;       // planes of a tile whose item offsets one wavefront's lanes hold
 
 constexpr int FFT_MAX_PASSES = 12;
