@@ -414,7 +414,7 @@ int setup_pme_tiles(pmx_ctx *c) {
   if (cap[0] == 0) auto_tile_caps(s, n, cap);
   int T[3];
   for (;;) {
-    for (int d = 0; d < 3; d++) T[d] = divisor_below(s.ngrid[d], cap[d]);
+    for (int d = 0; d < 3; d++) T[d] = divisor_below(s.ngrid[d], std::min(cap[d], PME_TILE_MAX));
     for (int d = 0; d < 3; d++) {
       a.K[d] = s.ngrid[d];
       a.T[d] = T[d];

@@ -136,8 +136,8 @@ struct PmeArgs {
   int *cnt;            // [P*nbin] items per bin; zero between calls
   int2 *kp;            // [nchrg*P] bin of an item and its place there
   // items sorted by bin, bead-major [P][nchrg]: fractional grid offsets and
-  // charge (4 values of the grid type), and (first support point per axis, 10
-  // bits each; charge index)
+  // charge (4 values of the grid type), and (first support point per axis in
+  // its tile, 10 bits each; charge index)
   void *rfs;
   int2 *ris;
   int *off;            // [P][nbin + 1] first sorted item of a bin
@@ -165,6 +165,7 @@ constexpr int EWALD_BLOCK = 256;
 constexpr int PME_NBIN_MAX = 1 << 17;  // bins of one bead
 constexpr long PME_MM_ITEMS = 100000;  // (charge, bead) items from which the matrix-core spread pays
 constexpr size_t OVERLAP_ITEMS = 60000;  // (site, bead) from which PME runs beside the mixed pair kernel
+constexpr int PME_TILE_MAX = 1 << 10;  // points of a tile along an axis: an item keeps its place there in 10 bits
 constexpr int PME_ZB_MAX = 63;       // planes of a tile whose item offsets one wavefront's lanes hold
 
 constexpr int FFT_MAX_PASSES = 12;

@@ -85,8 +85,9 @@ struct Rec<float> {
 
 // Item (charge ic, bead b): the fractional grid coordinates
 // (ewald3d_pme.c:241-262, 270-276), formed in FP64; the first support point
-// per axis, 10 bits each, with the charge's index; and the item's bin: its
-// tile and, with zb > 1, its plane within the tile.
+// per axis relative to its tile (below PME_TILE_MAX on a grid axis of any
+// length), 10 bits each, with the charge's index; and the item's bin: its tile
+// and, with zb > 1, its plane within the tile.
 template <typename T>
 __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typename Rec<T>::V &f, int2 &si) {
   const size_t ib = (size_t)a.ichrg[ic] * a.P + b;
@@ -96,7 +97,7 @@ __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typenam
   s[0] = x * hi[0] + y * hi[3] + z * hi[6];
   s[1] = x * hi[1] + y * hi[4] + z * hi[7];
   s[2] = x * hi[2] + y * hi[5] + z * hi[8];
-  int s0[3];
+  int tile[3], l[3];  // the tile along each axis, and the first support point in it
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const int K = a.K[d];
@@ -107,16 +108,17 @@ __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typenam
     // support points (0-based) ig - n + 1 .. ig, periodic; ig = K (a
     // coordinate rounding onto the upper face) is the same set as ig = 0
     ig = ((ig % K) + K) % K;
-    const int g = ig - a.n + 1;
-    s0[d] = ((g % K) + K) % K;
+    const int g = ig - a.n + 1, s0 = ((g % K) + K) % K;
+    tile[d] = s0 / a.T[d];
+    l[d] = s0 - tile[d] * a.T[d];
   }
   f.x = (T)fr[0];
   f.y = (T)fr[1];
   f.z = (T)fr[2];
   f.w = (T)a.q[a.ichrg[ic]];
-  si = make_int2(s0[0] | (s0[1] << 10) | (s0[2] << 20), ic);
-  const int tc = s0[2] / a.T[2], tile = (tc * a.nt[1] + s0[1] / a.T[1]) * a.nt[0] + s0[0] / a.T[0];
-  return a.zb > 1 ? tile * a.zb + s0[2] - tc * a.T[2] : tile;
+  si = make_int2(l[0] | (l[1] << 10) | (l[2] << 20), ic);
+  const int tl = (tile[2] * a.nt[1] + tile[1]) * a.nt[0] + tile[0];
+  return a.zb > 1 ? tl * a.zb + l[2] : tl;
 }
 
 // The counting sort of the items by bin.  k_pme_count: one thread per (charge,
@@ -276,14 +278,14 @@ __device__ __forceinline__ void tile_items(const PmeArgs &a, int tl, int b, int 
 // Weights of one item along the three axes: w[d][m] is the weight of support
 // point s_d + m (M_n index j = n - m); l[d] is s_d relative to the tile origin.
 template <int NI, bool DERIV, typename T>
-__device__ __forceinline__ void item_weights(const typename Rec<T>::V &f, int s, const int (&org)[3], T (&w)[3][NI],
-                                             T (&dw)[3][NI], int (&l)[3]) {
+__device__ __forceinline__ void item_weights(const typename Rec<T>::V &f, int s, T (&w)[3][NI], T (&dw)[3][NI],
+                                             int (&l)[3]) {
   const T fr[3] = {f.x, f.y, f.z};
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     T mn[NI + 1], dmn[NI + 1];
     bspline<NI, DERIV, T>(fr[d], mn, dmn);
-    l[d] = ((s >> (10 * d)) & 1023) - org[d];
+    l[d] = (s >> (10 * d)) & (PME_TILE_MAX - 1);
 #pragma unroll
     for (int m = 0; m < NI; m++) {
       w[d][m] = mn[NI - m];
@@ -316,8 +318,6 @@ __global__ void __launch_bounds__(64) k_pme_spread_mm(PmeArgs a) {
   int tl, b;
   xcd_unit_bead(a.ntile, a.P, tl, b);
   const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
-  int org[3];
-  tile_origin(a, tl, org[0], org[1], org[2]);
   const int Tz = a.T[2], H0 = a.H[0], H1 = a.H[1], H01 = H0 * H1;
   const int *off = a.off + (size_t)b * (a.nbin + 1) + (size_t)tl * Tz;
   const int offl = off[min(lane, Tz)];  // lane z holds the start of plane z's items (Tz < 64)
@@ -365,8 +365,8 @@ __global__ void __launch_bounds__(64) k_pme_spread_mm(PmeArgs a) {
 #pragma unroll
               for (int m = 0; m < NI; m++) sw[row][kq][m] = (double)mn[NI - m] * q;
             } else {
-              sl[row][0] = (sn & 1023) - org[0];
-              sl[row][1] = ((sn >> 10) & 1023) - org[1];
+              sl[row][0] = sn & (PME_TILE_MAX - 1);
+              sl[row][1] = (sn >> 10) & (PME_TILE_MAX - 1);
             }
             next(pb + NB);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -416,8 +416,6 @@ __global__ void __launch_bounds__(spread_lanes<T>() * PME_BLOCK) k_pme_spread(Pm
   tile_items(a, tl, b, lo, hi);
   const typename Rec<T>::V *rf = (const typename Rec<T>::V *)a.rfs + (size_t)b * a.nchrg;
   const int2 *ri = a.ris + (size_t)b * a.nchrg;
-  int org[3];
-  tile_origin(a, tl, org[0], org[1], org[2]);
   const int H0 = a.H[0], H01 = a.H[0] * a.H[1];
   __syncthreads();
   // L lanes per charge, each adding every L-th row (mc, mb) of the support
@@ -429,7 +427,7 @@ __global__ void __launch_bounds__(spread_lanes<T>() * PME_BLOCK) k_pme_spread(Pm
     const T q = f.w;
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, false, T>(f, ri[c].x, org, w, dw, l);
+    item_weights<NI, false, T>(f, ri[c].x, w, dw, l);
 #pragma unroll
     for (int m = 0; m < NI; m++) w[0][m] *= q;
     for (int rw = part; rw < NI * NI; rw += L) {
@@ -564,7 +562,7 @@ __global__ void __launch_bounds__(256) k_pme_gather(PmeArgs a) {
     const int i = a.ichrg[si.y];
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, true, T>(f, si.x, org, w, dw, l);
+    item_weights<NI, true, T>(f, si.x, w, dw, l);
     double wb[NI], dwb[NI];
 #pragma unroll
     for (int m = 0; m < NI; m++) {
@@ -643,7 +641,7 @@ __global__ void __launch_bounds__(PME_BLOCK) k_pme_phi(PmeArgs a) {
     const int i = a.ichrg[si.y];
     T w[3][NI], dw[3][NI];
     int l[3];
-    item_weights<NI, false, T>(rf[c], si.x, org, w, dw, l);
+    item_weights<NI, false, T>(rf[c], si.x, w, dw, l);
     double v = 0.0;
     for (int mc = 0; mc < NI; mc++) {
 #pragma unroll

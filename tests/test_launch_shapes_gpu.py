@@ -1,5 +1,7 @@
 """Force calls at the bead counts, grid sizes and box sizes where a kernel's
 launch shape or branch changes, against the oracle."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -195,3 +197,47 @@ def test_nve_steps_at_once(model, nmol, nsteps):
         assert abs(e0[k] - e1[k]) < FP64_TOL * scale, k
     assert k1 > 0 and abs(k0 - k1) < FP64_TOL * k1
     assert np.sqrt(((f0 - f1) ** 2).sum() / (f1 ** 2).sum()) < FP64_TOL
+
+
+def rod_config(axis, nmol, P, edge=5.0, length=975.0):
+    """Waters spread along a rod, its ends included: 1080 grid points along
+    axis and 8 along the others; P beads all at the same places."""
+    st = w.Settings(cutoff=2.4, skin=0.1, res_dist=2.0, rheal=0.5, alpha=3.5 / 2.4, kmax_ewd=8, kmax_pme=16)
+    c = w.build_config(w.SPC_FW, nmol, w.density_box(nmol), 1, 11, st)
+    e = np.full(3, edge)
+    e[axis] = length
+    to = np.random.default_rng(11).uniform(size=(nmol, 3)) * e
+    to[:, axis] = (np.arange(nmol) + 0.5) * length / nmol
+    x = np.stack([v.reshape(nmol, 3) for v in (c.x, c.y, c.z)], 2)
+    x += to[:, None] / w.BOHR - x[:, :1]
+    one = w.with_cell(w.Config(c.system, *(np.ascontiguousarray(x[..., d]).reshape(-1) for d in range(3))), np.diag(e))
+    beads = w.Config(dataclasses.replace(one.system, pi_beads=P), *(np.tile(v, P) for v in (one.x, one.y, one.z)))
+    return one, beads
+
+
+# grid axes past 1024 points, each axis in turn, the LDS and (10^5 items) the
+# matrix-core spread, and a tile asked to be as long as the axis.  Equal beads
+# have the energies of one, forces / P each.
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("axis, nmol, P, tile", [(0, 60, 1, None), (1, 60, 1, None), (2, 60, 1, None), (0, 530, 64, None),
+                                                 (1, 530, 64, None), (2, 530, 64, None), (2, 60, 1, "1,1,1080")])
+def test_pme_long_axis(monkeypatch, prec, axis, nmol, P, tile):
+    from piny_amd.engine import Engine
+    one, c = rod_config(axis, nmol, P)
+    if tile:
+        monkeypatch.setenv("PMX_PME_TILE", tile)
+        one.system.settings.n_interp = 4
+    o = Oracle(one.system, one.x, one.y, one.z)
+    assert sorted(o.scalars()[10:13]) == [8, 8, 1080]
+    eo, fo, _ = o.energy_control(one.x, one.y, one.z, 0)
+    eng = Engine(c.system, c.x, c.y, c.z, **({"precision": abi.PMX_PREC_MIXED} if prec == "mixed" else {}))
+    eng.set_positions(c.x, c.y, c.z)
+    e = eng.energy_control(abi.PMX_EVAL_PIMD if P > 1 else 0)
+    f = eng.forces() * P
+    eng.close()
+    etol, ftol = (FP64_TOL, FP64_TOL) if prec == "fp64" else (1e-5, 1e-4)
+    scale = max(abs(eo[k]) for k in abi.ENERGY_KEYS)
+    assert e["nver"] == eo["nver"]
+    for k in abi.ENERGY_KEYS:
+        assert abs(e[k] - eo[k]) < etol * scale, k
+    assert np.sqrt(((f - fo) ** 2).sum() / (P * (fo ** 2).sum())) < ftol
