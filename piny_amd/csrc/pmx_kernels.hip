@@ -551,13 +551,15 @@ __device__ __forceinline__ void list_record(const ListArgs &a, int d, int v) {
 // the counting sort's atomics leave them in arbitrary order), so that the
 // cell order, and the force-list order that follows it, is the same on
 // every build; then writes the sites' records in that order.  A cell of
-// more than CELL_SORT_MAX sites sets overflow[2] and the host builds with
-// the plain scan instead.
+// more than CELL_SORT_MAX sites sets overflow[2], and the host builds again
+// without cells; its records are written in the order they have, since the
+// row kernels are queued before the host reads the flag.
 __global__ void __launch_bounds__(256) k_cell_order(ListArgs a) {
   __shared__ int ids[CELL_SORT_MAX];
   const int c = blockIdx.x, n = a.cell_cnt[c], o = a.cell_start[c];
   if (n > CELL_SORT_MAX) {  // uniform over the workgroup
     if (threadIdx.x == 0) a.overflow[2] = 1;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) list_record(a, o + k, a.cell_sites[o + k]);
     return;
   }
   for (int k = threadIdx.x; k < n; k += blockDim.x) ids[k] = a.cell_sites[o + k];

@@ -138,6 +138,30 @@ def test_list_rows(monkeypatch, mode, nmol, P, cell):
     eng.close()
 
 
+# more sites in one cell than a workgroup orders, on a new context: the list
+# comes from the build without cells; then a call on spread positions
+@pytest.mark.parametrize("P", [1, 2])
+def test_list_of_an_overfull_cell(monkeypatch, P):
+    from piny_amd.engine import Engine
+    monkeypatch.setenv("PMX_LIST", "cells")
+    c = w.small_config(w.SPC_FW, nmol=700, P=P, seed=1, cutoff=3.0)
+    crowd = np.tile(np.arange(2100) < 1200, P)
+    x, y, z = (np.where(crowd, 2.0 + 0.02 * (v - v.mean()), v) for v in (c.x, c.y, c.z))
+    flags = abi.PMX_EVAL_PIMD if P > 1 else 0
+    eng = Engine(c.system, x, y, z)
+    o = Oracle(c.system, x, y, z)
+    for pos in ((x, y, z), (c.x, c.y, c.z)):
+        eng.set_positions(*pos)
+        e = eng.energy_control(flags)
+        eo, fo, _ = o.energy_control(*pos, flags)
+        assert e["nver"] == eo["nver"]
+        for a, b in zip(eng.verlet_list(), o.verlet_list()):
+            assert np.array_equal(a, b)
+    f = eng.forces()
+    assert np.sqrt(((f - fo) ** 2).sum() / (fo ** 2).sum()) < FP64_TOL
+    eng.close()
+
+
 # PME: a bead's sort in one workgroup and in three launches, the matrix-core
 # spread (10^5 items) and the LDS one, orders and grids with and without its
 # tiles, FP64 and mixed (the mixed bars of the parity tests)
