@@ -86,6 +86,31 @@ def test_pair_table_in_lds(nmol, P, nsplin):
     check(c)
 
 
+# two sites at one place, in every bead: a pair inside the cutoff, evaluated
+# past the start of its table, counted, and without a force of its own.  The
+# cubic reaches back over 82 points (0.1 A at 0.0012 A), with weights of up to
+# 82^3 / 2 = 3e5 on values rounded to 1e-16: 3e-11 of a table value.
+@pytest.mark.parametrize("P", [1, 2])
+@pytest.mark.parametrize("site", [0, 1])
+def test_pair_at_no_distance(monkeypatch, P, site):
+    from piny_amd.engine import Engine
+    c = w.small_config(w.SPC_FW, nmol=64, P=P, seed=5)
+    for v in (c.x, c.y, c.z):
+        v = v.reshape(P, 64, 3)
+        v[:, 7] += v[:, 3, site, None] - v[:, 7, site, None]
+        v[:, 7, site] = v[:, 3, site]
+    check(c)
+    npair = []
+    for mode in ("full", "half"):
+        monkeypatch.setenv("PMX_PAIR_LIST", mode)
+        eng = Engine(c.system, c.x, c.y, c.z)
+        eng.set_positions(c.x, c.y, c.z)
+        eng.energy_control()
+        npair.append(eng.pair_count())
+        eng.close()
+    assert npair[0] == npair[1]
+
+
 # Nose-Hoover chains: every length is a kernel of its own; the state against
 # the oracle's integrator
 @pytest.mark.parametrize("len_nhc", [1, 2, 3, 4, 5, 6, 7])
