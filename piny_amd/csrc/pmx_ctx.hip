@@ -3174,8 +3174,8 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
   int rc = PMX_OK;
   for (int step = 0; step < nsteps && !rc; step++) {
     hipLaunchKernelGGL(k_nhc_ckin, dim3(NHC_BLOCKS), dim3(256), 0, c->st, a);
-    (void)launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);  // errors: the check below
-    (void)launch_nhc(a, NHC_KICK0, 0, c->st);
+    launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);
+    launch_nhc(a, NHC_KICK0, 0, c->st);
     hipLaunchKernelGGL(k_mode_drift, dim3(mode_blocks(N, P)), dim3(256), 0, c->st, a);
     if (c->nghost)
       hipLaunchKernelGGL(k_ghost_pos, dim3(blocks((size_t)c->nghost * P)), dim3(256), 0, c->st, c->nghost, P,
@@ -3185,9 +3185,9 @@ int pmx_pimd_nvt(pmx_ctx *c, const pmx_nhc_params *np, int nsteps, pmx_energies 
       break;
     }
     if ((rc = step_force(c, flags))) break;
-    (void)launch_nhc(a, NHC_KICK1, 0, c->st);
+    launch_nhc(a, NHC_KICK1, 0, c->st);
     hipLaunchKernelGGL(k_nhc_ckin, dim3(NHC_BLOCKS), dim3(256), 0, c->st, a);
-    (void)launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);
+    launch_nhc(a, NHC_CLASS, NHC_BLOCKS, c->st);
     hipLaunchKernelGGL(k_nhc_scale0, dim3(gN), dim3(256), 0, c->st, a);
   }
   c->xmod_given = xmod_given;

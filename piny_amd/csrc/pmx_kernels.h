@@ -311,9 +311,10 @@ struct NhcArgs {
   double *x, *y, *z, *xm, *ym, *zm;
 };
 __global__ void k_nhc_ckin(NhcArgs a);
-// the centroid chain over G partial sums, or the chains and kick of a half step
+// the centroid chain over G partial sums, or the chains and kick of a half
+// step; a failed launch is left for the caller's hipGetLastError
 enum { NHC_CLASS, NHC_KICK0, NHC_KICK1 };
-hipError_t launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st);
+void launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st);
 __global__ void k_nhc_scale0(NhcArgs a);
 __global__ void k_mode_drift(NhcArgs a);
 __global__ void k_pimd_energy(NhcArgs a);

@@ -3316,7 +3316,7 @@ static void launch_nhc_len(const NhcArgs &a, int what, int G, hipStream_t st) {
                        what == NHC_KICK1 ? 1 : 0);
 }
 
-hipError_t launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st) {
+void launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st) {
   switch (a.len) {
     case 1: launch_nhc_len<1>(a, what, G, st); break;
     case 2: launch_nhc_len<2>(a, what, G, st); break;
@@ -3326,7 +3326,6 @@ hipError_t launch_nhc(const NhcArgs &a, int what, int G, hipStream_t st) {
     case 6: launch_nhc_len<6>(a, what, G, st); break;
     default: launch_nhc_len<7>(a, what, G, st); break;  // the length is checked to be 1..7
   }
-  return hipGetLastError();
 }
 
 // the centroid mode's velocities scaled by its chain's factor (phase 1)
