@@ -87,6 +87,7 @@ struct pmx_ctx {
   int *site_cell = nullptr, *site_pos = nullptr, *cell_cnt = nullptr, *cell_start = nullptr, *cell_sites = nullptr;
   bool list_cells = false;  // the last build used link cells
   bool ref_valid = false;   // jfull / nfull hold the reference's half list of the last build
+  int ref_cap = 0;          // width of jfull's rows
   double *xm0 = nullptr, *ym0 = nullptr, *zm0 = nullptr;  // xmod at the last build
   PairTypes pt_build{};     // cut+skin at the last build
   double4 *cell_p = nullptr, *cell_m = nullptr;  // sites in cell order (link-cell build)
@@ -301,17 +302,15 @@ int alloc_lists(pmx_ctx *c, int cap) {
                "one call of pmx_energy_control grows them", cap, c->cap);
     return PMX_ERR_RANGE;
   }
-  if (c->jfull) {
-    for (int *p : {c->jfull, c->jforce, c->jsplit}) {
-      (void)hipFree(p);
-      c->allocs.erase(std::remove(c->allocs.begin(), c->allocs.end(), (void *)p), c->allocs.end());
-    }
-  }
-  c->cap = cap;
+  dfree(c, c->jfull);
+  dfree(c, c->jforce);
+  dfree(c, c->jsplit);
+  c->cap = c->ref_cap = 0;  // no rows, should an allocation fail
   c->epoch++;
   int rc = dalloc(c, &c->jfull, n);
   if (!rc) rc = dalloc(c, &c->jforce, n);
   if (!rc) rc = dalloc(c, &c->jsplit, n);
+  if (!rc) c->cap = c->ref_cap = cap;
   return rc;
 }
 
@@ -1390,7 +1389,8 @@ int build_list(pmx_ctx *c) {
 
 // The reference's half list in its order (verlist_create.c:373-503), from
 // the positions, xmod and cut+skin of the last build, by the ascending scan
-// over j < i.
+// over j < i.  Its rows hold pairs that do not interact too, and one can be
+// longer than the force list's longest: they then get a width of their own.
 int build_ref_list(pmx_ctx *c) {
   ListArgs a = list_args(c);
   a.bx = c->x0;
@@ -1402,13 +1402,23 @@ int build_ref_list(pmx_ctx *c) {
   a.pt = c->pt_build;
   a.full = 0;
   a.ref_only = 1;
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->st, c->overflow, 0, (size_t)4);
-  hipLaunchKernelGGL(k_list_build, dim3(blocks((size_t)c->s.N * 64)), dim3(256), 0, c->st, a);
-  hipLaunchKernelGGL(k_list_counts, dim3(1), dim3(1024), 0, c->st, a);
-  HIPCHK(hipGetLastError());
-  int ov[4];
-  HIPCHK(hipMemcpyAsync(ov, c->overflow, sizeof ov, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
+  int ov[4] = {0, -1, 0, 0};
+  for (int attempt = 0; attempt < 2; attempt++) {
+    a.jfull = c->jfull;
+    a.cap = c->ref_cap;
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->st, c->overflow, 0, (size_t)4);
+    hipLaunchKernelGGL(k_list_build, dim3(blocks((size_t)c->s.N * 64)), dim3(256), 0, c->st, a);
+    hipLaunchKernelGGL(k_list_counts, dim3(1), dim3(1024), 0, c->st, a);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(ov, c->overflow, sizeof ov, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    if (ov[0] == 0) break;
+    const int want = ((ov[0] + 63) / 64) * 64;
+    dfree(c, c->jfull);
+    c->ref_cap = 0;  // no rows, should the allocation fail
+    TRY_RC(dalloc(c, &c->jfull, (size_t)c->s.N * want));
+    c->ref_cap = want;
+  }
   if (ov[0] != 0 || ov[1] != c->nver) {
     set_err(c, "reference list rebuild: %d pairs against %d of the force list's build", ov[1], c->nver);
     return PMX_ERR_STATE;
@@ -3567,10 +3577,9 @@ int pmx_get_verlet_list(pmx_ctx *c, int *nter, int *jver_off, int *jter, int cap
   }
   *nver = (int)tot;
   if (cap < tot || !jter) return cap < tot ? PMX_ERR_RANGE : PMX_OK;
-  std::vector<int> row(c->cap);
   for (int i = 0; i < N; i++) {
     if (nter[i] == 0) continue;
-    HIPCHK(hipMemcpy(jter + jver_off[i], c->jfull + (size_t)i * c->cap, nter[i] * sizeof(int),
+    HIPCHK(hipMemcpy(jter + jver_off[i], c->jfull + (size_t)i * c->ref_cap, nter[i] * sizeof(int),
                      hipMemcpyDeviceToHost));
   }
   return PMX_OK;

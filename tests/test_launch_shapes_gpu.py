@@ -187,6 +187,25 @@ def test_list_of_an_overfull_cell(monkeypatch, P):
     eng.close()
 
 
+# a crowd of sites of which not all interact (the oxygens of q-TIP4P/F have no
+# charge): the reference's longest row is longer than the force list's
+@pytest.mark.parametrize("mode", ["brute", "cells"])
+def test_reference_list_of_a_crowd(monkeypatch, mode):
+    from piny_amd.engine import Engine
+    monkeypatch.setenv("PMX_LIST", mode)
+    c = w.small_config(w.Q_TIP4P_F, nmol=230, seed=1, box=60.0, cutoff=5.0)
+    x, y, z = (0.1 * (v - v.mean()) for v in (c.x, c.y, c.z))
+    eng = Engine(c.system, x, y, z)
+    eng.set_positions(x, y, z)
+    e = eng.energy_control(0)
+    o = Oracle(c.system, x, y, z)
+    eo, _, _ = o.energy_control(x, y, z, 0)
+    assert e["nver"] == eo["nver"]
+    for a, b in zip(eng.verlet_list(), o.verlet_list()):
+        assert np.array_equal(a, b)
+    eng.close()
+
+
 # PME: a bead's sort in one workgroup and in three launches, the matrix-core
 # spread (10^5 items) and the LDS one, orders and grids with and without its
 # tiles, FP64 and mixed (the mixed bars of the parity tests)
