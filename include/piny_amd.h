@@ -451,7 +451,8 @@ int pmx_autotune(pmx_ctx *ctx, unsigned flags, int reps, int *choice);
 /* The autotuner for a batch: the boxes share the device, so candidates are
  * timed as whole batched calls, each applied to every context: the pair
  * kernels' wavefront cap, then the PME tile caps.  choice (may be NULL)
- * receives [pair wavefronts, tile cap a, b, c].  Ends with a batched call. */
+ * receives [pair wavefronts, tile cap a, b, c] (caps 0, 0, 0: chosen per box).
+ * Ends with a batched call. */
 int pmx_batch_autotune(pmx_batch *batch, unsigned flags, int reps, int *choice);
 
 /* Coefficient helpers restating intra_coefs.c (units: Hartree, Bohr). */

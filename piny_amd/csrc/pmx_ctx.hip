@@ -160,7 +160,7 @@ struct pmx_ctx {
   // launch shapes (set at creation, changed by pmx_autotune): PME tile
   // caps, wavefronts of the pair kernels, list build (0 by size, 1 plain
   // scan, 2 link cells)
-  int tile_cap[3] = {0, 0, 0};  // upper bounds of the PME tile; 0: auto_tile_caps
+  int tile_cap[3] = {0, 0, 0};  // upper bounds of the PME tile; all 0: auto_tile_caps
   int pair_waves = 4096;
   int list_mode = 0;
   hipEvent_t ready = nullptr;  // list stage done (batched calls)
@@ -410,7 +410,7 @@ int setup_pme_tiles(pmx_ctx *c) {
     return t;
   };
   int cap[3] = {c->tile_cap[0], c->tile_cap[1], c->tile_cap[2]};
-  if (cap[0] == 0) auto_tile_caps(s, n, cap);
+  if (cap[0] == 0 && cap[1] == 0 && cap[2] == 0) auto_tile_caps(s, n, cap);
   int T[3];
   for (;;) {
     for (int d = 0; d < 3; d++) T[d] = divisor_below(s.ngrid[d], std::min(cap[d], PME_TILE_MAX));
@@ -2238,8 +2238,10 @@ pmx_ctx *pmx_create(const pmx_system *sys, const pmx_params *par, const double *
   if (const char *env = getenv("PMX_CLUSTER")) c->clu_enabled = atoi(env) == 1;
   if (const char *env = getenv("PMX_PAIR_WAVES"))  // tuning override: wavefronts of the pair kernels
     c->pair_waves = std::max(64, std::min(PAIR_MAX_WAVES, atoi(env)));
-  if (const char *env = getenv("PMX_PME_TILE"))  // tuning override "Ta,Tb,Tc" (upper bounds)
-    sscanf(env, "%d,%d,%d", &c->tile_cap[0], &c->tile_cap[1], &c->tile_cap[2]);
+  if (const char *env = getenv("PMX_PME_TILE")) {  // tuning override "Ta,Tb,Tc" (upper bounds; 16, 16, 8 if left out)
+    int cap[3] = {16, 16, 8};
+    if (sscanf(env, "%d,%d,%d", &cap[0], &cap[1], &cap[2]) >= 1) std::copy(cap, cap + 3, c->tile_cap);
+  }
   if (build_device(c, sys) != PMX_OK) {
     std::string e = c->err;
     pmx_destroy(c);

@@ -2,7 +2,8 @@
  * front of libamdhip64 by LD_PRELOAD: memory is host memory, copies are
  * memcpy, streams and events do nothing, kernels are not run.  fake_fail(name,
  * n) makes the n-th launch from then on of the kernels whose (mangled) name
- * holds name fail: the error stays until hipGetLastError takes it. */
+ * holds name fail: the error stays until hipGetLastError takes it.
+ * fake_grid(name): workgroups along x of their last launch. */
 #include <stdlib.h>
 #include <string.h>
 
@@ -10,6 +11,7 @@ enum { MAX_KERNELS = 4096, LAUNCH_FAILED = 719 };
 static struct {
   const void *host;
   const char *name;
+  unsigned grid;
 } kernels[MAX_KERNELS];
 static int nkernel, last, fail_at, token;
 static char fail_name[64];
@@ -20,10 +22,24 @@ void fake_fail(const char *name, int n) {
   last = 0;
 }
 
-int hipLaunchKernel(const void *f) {
+unsigned fake_grid(const char *name) {
+  for (int k = 0; k < nkernel; k++)
+    if (kernels[k].grid && strstr(kernels[k].name, name)) return kernels[k].grid;
+  return 0;
+}
+
+struct dim3 {
+  unsigned x, y, z;
+};
+static struct dim3 grid_pushed;
+int __hipPushCallConfiguration(struct dim3 grid) { return grid_pushed = grid, 0; }
+int __hipPopCallConfiguration(struct dim3 *grid) { return *grid = grid_pushed, 0; }
+int hipLaunchKernel(const void *f, struct dim3 grid) {
   int k;
   for (k = 0; k < nkernel && kernels[k].host != f;) k++;
-  if (k < nkernel && fail_at > 0 && strstr(kernels[k].name, fail_name) && --fail_at == 0) return last = LAUNCH_FAILED;
+  if (k == nkernel) return 0;
+  if (fail_at > 0 && strstr(kernels[k].name, fail_name) && --fail_at == 0) return last = LAUNCH_FAILED;
+  kernels[k].grid = grid.x;
   return 0;
 }
 int hipGetLastError(void) {
@@ -42,8 +58,6 @@ void __hipRegisterFunction(void **m, const void *host, char *device, const char 
 }
 void __hipRegisterVar(void) {}
 void __hipUnregisterFatBinary(void) {}
-int __hipPushCallConfiguration(void) { return 0; }
-int __hipPopCallConfiguration(void) { return 0; }
 
 static int alloc(void **p, size_t n) { return (*p = calloc(1, n ? n : 1)) ? 0 : 2; }
 int hipMalloc(void **p, size_t n) { return alloc(p, n); }
