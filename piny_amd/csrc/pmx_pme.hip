@@ -87,9 +87,12 @@ struct Rec<float> {
 // (ewald3d_pme.c:241-262, 270-276), formed in FP64; the first support point
 // per axis relative to its tile (below PME_TILE_MAX on a grid axis of any
 // length), 10 bits each, with the charge's index; and the item's bin: its tile
-// and, with zb > 1, its plane within the tile.
+// and, with zb > 1, its plane within the tile.  No contraction: k_pme_count and
+// k_pme_place form the same item, and both must round alike for the bin that
+// the one counted to be the other's.
 template <typename T>
 __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typename Rec<T>::V &f, int2 &si) {
+#pragma clang fp contract(off)
   const size_t ib = (size_t)a.ichrg[ic] * a.P + b;
   const double x = a.x[ib], y = a.y[ib], z = a.z[ib];
   const double *hi = a.cell.hi;
