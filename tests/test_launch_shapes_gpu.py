@@ -267,6 +267,30 @@ def test_nve_steps_at_once(model, nmol, nsteps):
     assert np.sqrt(((f0 - f1) ** 2).sum() / (f1 ** 2).sum()) < FP64_TOL
 
 
+def equal_beads(one, P):
+    """The one-bead configuration with P beads at its places."""
+    return w.Config(dataclasses.replace(one.system, pi_beads=P), *(np.tile(v, P) for v in (one.x, one.y, one.z)))
+
+
+def check_equal_beads(one, c, prec):
+    """The call on P equal beads has the energies of one bead, and its forces
+    / P on each."""
+    from piny_amd.engine import Engine
+    P = c.system.pi_beads
+    eo, fo, _ = Oracle(one.system, one.x, one.y, one.z).energy_control(one.x, one.y, one.z, 0)
+    eng = Engine(c.system, c.x, c.y, c.z, precision=abi.PMX_PREC_MIXED if prec == "mixed" else abi.PMX_PREC_FP64)
+    eng.set_positions(c.x, c.y, c.z)
+    e = eng.energy_control(abi.PMX_EVAL_PIMD if P > 1 else 0)
+    f = eng.forces() * P
+    eng.close()
+    etol, ftol = (FP64_TOL, FP64_TOL) if prec == "fp64" else (1e-5, 1e-4)
+    scale = max(abs(eo[k]) for k in abi.ENERGY_KEYS)
+    assert e["nver"] == eo["nver"]
+    for k in abi.ENERGY_KEYS:
+        assert abs(e[k] - eo[k]) < etol * scale, k
+    assert np.sqrt(((f - fo) ** 2).sum() / (P * (fo ** 2).sum())) < ftol
+
+
 def rod_config(axis, nmol, P, edge=5.0, length=975.0):
     """Waters spread along a rod, its ends included: 1080 grid points along
     axis and 8 along the others; P beads all at the same places."""
@@ -279,33 +303,44 @@ def rod_config(axis, nmol, P, edge=5.0, length=975.0):
     x = np.stack([v.reshape(nmol, 3) for v in (c.x, c.y, c.z)], 2)
     x += to[:, None] / w.BOHR - x[:, :1]
     one = w.with_cell(w.Config(c.system, *(np.ascontiguousarray(x[..., d]).reshape(-1) for d in range(3))), np.diag(e))
-    beads = w.Config(dataclasses.replace(one.system, pi_beads=P), *(np.tile(v, P) for v in (one.x, one.y, one.z)))
-    return one, beads
+    return one, equal_beads(one, P)
 
 
 # grid axes past 1024 points, each axis in turn, the LDS and (10^5 items) the
-# matrix-core spread, and a tile asked to be as long as the axis.  Equal beads
-# have the energies of one, forces / P each.
+# matrix-core spread, and a tile asked to be as long as the axis
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("axis, nmol, P, tile", [(0, 60, 1, None), (1, 60, 1, None), (2, 60, 1, None), (0, 530, 64, None),
                                                  (1, 530, 64, None), (2, 530, 64, None), (2, 60, 1, "1,1,1080")])
 def test_pme_long_axis(monkeypatch, prec, axis, nmol, P, tile):
-    from piny_amd.engine import Engine
     one, c = rod_config(axis, nmol, P)
     if tile:
         monkeypatch.setenv("PMX_PME_TILE", tile)
         one.system.settings.n_interp = 4
-    o = Oracle(one.system, one.x, one.y, one.z)
-    assert sorted(o.scalars()[10:13]) == [8, 8, 1080]
-    eo, fo, _ = o.energy_control(one.x, one.y, one.z, 0)
-    eng = Engine(c.system, c.x, c.y, c.z, **({"precision": abi.PMX_PREC_MIXED} if prec == "mixed" else {}))
-    eng.set_positions(c.x, c.y, c.z)
-    e = eng.energy_control(abi.PMX_EVAL_PIMD if P > 1 else 0)
-    f = eng.forces() * P
-    eng.close()
-    etol, ftol = (FP64_TOL, FP64_TOL) if prec == "fp64" else (1e-5, 1e-4)
-    scale = max(abs(eo[k]) for k in abi.ENERGY_KEYS)
-    assert e["nver"] == eo["nver"]
-    for k in abi.ENERGY_KEYS:
-        assert abs(e[k] - eo[k]) < etol * scale, k
-    assert np.sqrt(((f - fo) ** 2).sum() / (P * (fo ** 2).sum())) < ftol
+    assert sorted(Oracle(one.system, one.x, one.y, one.z).scalars()[10:13]) == [8, 8, 1080]
+    check_equal_beads(one, c, prec)
+
+
+# grids that are not cubes, under the matrix-core spread (10^5 items) and the
+# LDS one: tiles wider along a than along b and the reverse, odd ones, and a
+# triclinic cell
+SHEAR = ((1.0, 0.15, 0.0), (0.0, 1.0, 0.1), (0.05, 0.0, 1.0))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("P", [64, 2])
+@pytest.mark.parametrize("grid, order, shear", [((48, 48, 64), 6, None), ((48, 40, 64), 6, None), ((36, 48, 40), 6, None),
+                                                ((40, 36, 48), 8, None), ((48, 40, 36), 4, None), ((36, 40, 64), 6, SHEAR)])
+def test_pme_grids_not_cubic(prec, P, grid, order, shear):
+    nmol = 530
+    k = np.array(grid) / 4 - 1
+    kpme = round(2 * k.prod() ** (1 / 3))
+    st = w.Settings(cutoff=2.5, skin=0.5, alpha=1.0, kmax_ewd=8, kmax_pme=kpme, n_interp=order)
+    L = w.density_box(nmol)
+    c = w.build_config(w.SPC_FW, nmol, L, 1, 21, st)
+    cell = np.diag(L * k / k.prod() ** (1 / 3)) @ np.array(shear or np.eye(3))
+    # molecules at the fractions of the cell that they have of the cube
+    x = np.stack([v.reshape(nmol, 3) for v in (c.x, c.y, c.z)], 2)
+    x += (x[:, :1] * w.BOHR / L) @ cell.T / w.BOHR - x[:, :1]
+    one = w.with_cell(w.Config(c.system, *(np.ascontiguousarray(x[..., d]).reshape(-1) for d in range(3))), cell)
+    assert tuple(Oracle(one.system, one.x, one.y, one.z).scalars()[10:13]) == grid
+    check_equal_beads(one, equal_beads(one, P), prec)
