@@ -1259,8 +1259,11 @@ int build_device(pmx_ctx *c, const pmx_system *sys) {
 // for either or the cells spare a site fewer than 6000 candidates: their
 // sorting is five launches more (list stage of a rebuild without and with
 // cells: 144 and 155 us at 8000 sites, 5100 candidates spared; 226 and 200 us
-// at 12000, 9900 spared; 305 and 216 us at 16384).  PMX_LIST=brute|cells and
-// the autotuner choose otherwise.
+// at 12000, 9900 spared; 305 and 216 us at 16384).  In a triclinic cell every
+// candidate takes the FP64 test, and 2000 spared pay for the sorting (110 and
+// 120 us at 3000 sites, 1260 spared; 155 and 143 at 4200, 2120 spared; 219 and
+// 154 at 6000, 4090 spared; 335 and 204 at 8100, 5800 spared).
+// PMX_LIST=brute|cells and the autotuner choose otherwise.
 int choose_cells(const pmx_ctx *c, int nc[3]) {
   const char *env = getenv("PMX_LIST");  // tuning override: "brute" or "cells"
   if ((env && strcmp(env, "brute") == 0) || c->list_mode == 1) return 0;
@@ -1278,7 +1281,7 @@ int choose_cells(const pmx_ctx *c, int nc[3]) {
     }
     if (!ok || ncell > (size_t)MAX_LIST_CELLS) continue;
     const double spared = (double)c->s.N * (1.0 - (2 * H + 1) * (2 * H + 1) * (2 * H + 1) / (double)ncell);
-    return env || c->list_mode == 2 || spared >= 6000.0 ? H : 0;
+    return env || c->list_mode == 2 || spared >= (c->cell.cubic ? 6000.0 : 2000.0) ? H : 0;
   }
   return 0;
 }

@@ -38,6 +38,15 @@ eng.set_positions(c.x, c.y, c.z)
 eng.energy_control()
 print(fake.fake_grid(b"k_pme_gather"))
 """
+CELLS = SETUP + """
+nmol, cell = int(sys.argv[1]), np.array(eval(sys.argv[2]))
+L = w.density_box(nmol)
+c = w.build_config(w.SPC_FW, nmol, L, 1, 1, w.Settings(kmax_ewd=10, kmax_pme=10))
+eng = Engine(w.with_cell(c, cell / np.linalg.det(cell) ** (1 / 3) * L).system)
+eng.set_positions(c.x, c.y, c.z)
+eng.energy_control()
+print(fake.fake_grid(b"k_cell_order") > 0)
+"""
 
 
 @pytest.fixture(scope="module")
@@ -73,3 +82,15 @@ def test_pme_tile_override(run, tile, ntile):
         ntile = int(run(TILES))
         assert ntile != 2 * 2 * 4
     assert int(run(TILES, PMX_PME_TILE=tile)) == ntile
+
+
+# the list is built by cells where they spare a site 6000 candidates, 2000 in
+# a triclinic cell
+HEXAGONAL = "((1.0, 0.5, 0.0), (0.0, 0.866, 0.0), (0.0, 0.0, 1.0))"
+
+
+@pytest.mark.parametrize("nmol, cell, cells", [(2000, "np.eye(3)", False), (4000, "np.eye(3)", True),
+                                               (1000, HEXAGONAL, False), (2000, HEXAGONAL, True),
+                                               (2700, HEXAGONAL, True)])
+def test_list_cells_rule(run, nmol, cell, cells):
+    assert run(CELLS, str(nmol), cell).split() == [str(cells)]
