@@ -244,27 +244,31 @@ def test_fft_sizes(prec, K):
 
 
 # the kernel between two force calls of the NVE integrator: one step (no half
-# kick before), and several at once against the same steps one at a time,
+# kick before), and several at once, one at a time and by the oracle's forces,
 # with sites of a whole workgroup, of one more, and with ghosts
 @pytest.mark.parametrize("model, nmol, nsteps", [(w.SPC_FW, 64, 1), (w.SPC_FW, 64, 2), (w.Q_TIP4P_F, 65, 5),
                                                  (w.SPC_FW, 86, 7)])
 def test_nve_steps_at_once(model, nmol, nsteps):
     from piny_amd.engine import Engine
+    from tests.test_md_nve import oracle_nve
     c = w.small_config(model, nmol=nmol, P=1, seed=nmol)
     out = []
+    dt = 0.25 / abi.TIME_CONV
     for calls in ([nsteps], [1] * nsteps):
         eng = Engine(c.system, c.x, c.y, c.z)
         eng.set_positions(c.x, c.y, c.z)
         for n in calls:
-            e, ke = eng.md_nve(n, 0.25 / abi.TIME_CONV)
-        out.append((e, ke, eng.forces()))
+            e, ke = eng.md_nve(n, dt)
+        out.append((e, ke, eng.positions()[0], eng.velocities()[0], eng.forces()[0]))
         eng.close()
-    (e0, k0, f0), (e1, k1, f1) = out
+    e1, k1, x1, v1, f1 = oracle_nve(c, np.zeros((c.system.natm, 3)), nsteps, dt)
     scale = max(abs(e1[k]) for k in abi.ENERGY_KEYS)
-    for k in abi.ENERGY_KEYS:
-        assert abs(e0[k] - e1[k]) < FP64_TOL * scale, k
-    assert k1 > 0 and abs(k0 - k1) < FP64_TOL * k1
-    assert np.sqrt(((f0 - f1) ** 2).sum() / (f1 ** 2).sum()) < FP64_TOL
+    for e0, k0, x0, v0, f0 in out:
+        for k in abi.ENERGY_KEYS:
+            assert abs(e0[k] - e1[k]) < FP64_TOL * scale, k
+        assert k1 > 0 and abs(k0 - k1) < FP64_TOL * k1
+        for a, b in ((x0, x1), (v0, v1), (f0, f1)):
+            assert np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum()) < FP64_TOL
 
 
 def equal_beads(one, P):
