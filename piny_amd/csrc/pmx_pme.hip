@@ -87,9 +87,11 @@ struct Rec<float> {
 // (ewald3d_pme.c:241-262, 270-276), formed in FP64; the first support point
 // per axis relative to its tile (below PME_TILE_MAX on a grid axis of any
 // length), 10 bits each, with the charge's index; and the item's bin: its tile
-// and, with zb > 1, its plane within the tile.  No contraction: k_pme_count and
-// k_pme_place form the same item, and both must round alike for the bin that
-// the one counted to be the other's.
+// and, with zb > 1, its plane within the tile.  The fused operations are written
+// out and no others formed: k_pme_count and k_pme_place form the same item, and
+// both must round alike for the bin that the one counted to be the other's.
+// (Without them k_pme_count takes 33 VGPRs and no longer fits beside the mixed
+// pair kernel's four wavefronts of 120: 12001 SPC/Fw, P = 16, 689 -> 705 us.)
 template <typename T>
 __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typename Rec<T>::V &f, int2 &si) {
 #pragma clang fp contract(off)
@@ -97,9 +99,9 @@ __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typenam
   const double x = a.x[ib], y = a.y[ib], z = a.z[ib];
   const double *hi = a.cell.hi;
   double s[3], fr[3];
-  s[0] = x * hi[0] + y * hi[3] + z * hi[6];
-  s[1] = x * hi[1] + y * hi[4] + z * hi[7];
-  s[2] = x * hi[2] + y * hi[5] + z * hi[8];
+  s[0] = fma(z, hi[6], fma(y, hi[3], x * hi[0]));
+  s[1] = fma(z, hi[7], fma(y, hi[4], x * hi[1]));
+  s[2] = fma(z, hi[8], fma(y, hi[5], x * hi[2]));
   int tile[3], l[3];  // the tile along each axis, and the first support point in it
 #pragma unroll
   for (int d = 0; d < 3; d++) {
@@ -107,7 +109,7 @@ __device__ __forceinline__ int pme_item(const PmeArgs &a, int ic, int b, typenam
     const double t = s[d] - nint_d((s[d] - 0.5));
     const double sc = t * (double)K;
     int ig = (int)(sc);
-    fr[d] = sc - (double)ig;
+    fr[d] = fma(t, (double)K, -(double)ig);
     // support points (0-based) ig - n + 1 .. ig, periodic; ig = K (a
     // coordinate rounding onto the upper face) is the same set as ig = 0
     ig = ((ig % K) + K) % K;
