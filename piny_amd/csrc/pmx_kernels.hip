@@ -607,8 +607,9 @@ __device__ __forceinline__ void wave_sync() {
 //
 // A workgroup per cell with the FP64 test for every candidate, staged in LDS
 // a stencil row at a time, had 125 workgroups for 1024 q-TIP4P/F at P = 8 and
-// 320 us of kernel for 4096 of them at 31 % VALU busy.  The list stage of a
-// rebuilding call, before -> now: 671 -> 105 us and 429 -> 216 us.
+// 320 us of kernel for 4096 of them at 31 % VALU busy (now 143 us at 70 %).
+// The list stage of a rebuilding call, before -> now: 671 -> 105 us and 429 ->
+// 216 us.
 constexpr int LIST_WAVES = 4;
 template <int H>
 __global__ void __launch_bounds__(64 * LIST_WAVES) k_list_rows(ListArgs a) {
@@ -1577,10 +1578,12 @@ __device__ __forceinline__ double sqrt_normal(double x) {
 // table's gathers were the bound: every lane of a term takes 64 bytes at its
 // own place of a table larger than the L1, about 180 bytes of lines each
 // (4096 q-TIP4P/F, P = 32: 911 us at 47 % VALU busy, 785 us with the table
-// in LDS).  The kernel then issues FP64 instructions: 109 a term, of which
-// the correctly rounded root, the interpolation's coefficients per function,
-// 64-bit addresses and the index's integer round trip were 40 (spline4_both,
-// sqrt_normal, byte offsets staged with the entries): 540 us.
+// in LDS).  Of the 109 FP64 instructions a term, the correctly rounded root,
+// the interpolation's coefficients per function, 64-bit addresses and the
+// index's integer round trip were 40 (spline4_both, sqrt_normal, byte offsets
+// staged with the entries): 540 us.  Now the vector units are busy 58 % and LDS
+// 37 % of the cycles, nearly half of that bank conflicts of the table reads:
+// four wavefronts a SIMD do not cover a term's chain.
 //
 // a.wps wavefronts share a site, taking its row's chunks in turn, and add
 // their forces through LDS: with fewer sites than the 4096 wavefronts the

@@ -535,9 +535,9 @@ __device__ __forceinline__ void load_halo_rows(const PmeArgs &a, int b, const in
 // mc = part * NI / 2 ... and the pair adds its sums.  Row sums in T; their
 // products with the other axes' weights and the sums over rows in FP64.  V:
 // points a lane loads (load_halo_rows), 0 for tiles it does not take.
-// 4096 q-TIP4P/F at P = 32, mixed 35 -> 26 us, FP64 47 -> 40 us (its LDS
-// reads are three quarters of that, the other half of the bank conflicts being
-// the charges' random places).
+// 4096 q-TIP4P/F at P = 32, mixed 35 -> 26 us, FP64 47 -> 40 us (LDS busy 59 %
+// of the cycles, half of that bank conflicts of the charges' random places;
+// vector units 49 %).
 template <int NI, typename T, int V>
 __global__ void __launch_bounds__(256) k_pme_gather(PmeArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
